@@ -124,15 +124,12 @@ struct FQ8_0 {
 
 // get_scale_min_k4 (quantized/utils.rs:50-60) for sub-block j of a Q4_K / Q5_K super-block whose
 // first 16 bytes (d, dmin, the 12 scale bytes) are hd
-__device__ __forceinline__ uint32_t k4_sbyte(const uint4 &hd, int i) { return ((&hd.x)[1 + (i >> 2)] >> (8 * (i & 3))) & 0xFF; }
+// (selects on the three dwords: an index into them that depends on j would put hd in scratch memory)
 __device__ __forceinline__ void k4_sc_mn(const uint4 &hd, int j, uint32_t &sc, uint32_t &mn) {
-    if (j < 4) {
-        sc = k4_sbyte(hd, j) & 63;
-        mn = k4_sbyte(hd, j + 4) & 63;
-    } else {
-        sc = (k4_sbyte(hd, j + 4) & 0xF) | ((k4_sbyte(hd, j - 4) >> 6) << 4);
-        mn = (k4_sbyte(hd, j + 4) >> 4) | ((k4_sbyte(hd, j) >> 6) << 4);
-    }
+    const int sh = 8 * (j & 3);
+    const uint32_t b0 = (hd.y >> sh) & 0xFF, b1 = (hd.z >> sh) & 0xFF, b2 = (hd.w >> sh) & 0xFF;
+    sc = j < 4 ? b0 & 63 : (b2 & 0xF) | ((b0 >> 6) << 4);
+    mn = j < 4 ? b1 & 63 : (b2 >> 4) | ((b1 >> 6) << 4);
 }
 
 // ---------------------------------------------------------------------------------- Q4_K

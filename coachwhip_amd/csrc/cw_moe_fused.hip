@@ -1,15 +1,13 @@
 // The MoE layer in two kernels (gfx950):
 //
-//  k_moe_gateup: every wavefront routes its token (softmax + top-k, cw_wave.h), looks its pick's
-//    slot up (identity, or the bank's slot table), and computes rows of gate and up for that
-//    pick with the activation fused: h = silu(g) * u, or gpt-oss's clamped SwiGLU with biases.
-//    The first block of each pick also publishes (expert, weight, slot) for the down kernel.
-//  k_moe_down: a tile of output rows of one token, every pick; waves split the picks, each
-//    pick's dots land in LDS and are combined in pick order (deterministic), with down's bias.
+//  k_moe_gateup: blocks of one token: one wave routes it (softmax + top-k, cw_wave.h) and looks the
+//    picks' slots up (identity, or the bank's slot table); the waves compute rows of gate and up of
+//    the picks with the activation fused: h = silu(g) * u, or gpt-oss's clamped SwiGLU with biases.
+//    The first block of each token also publishes (expert, weight, slot) for the down kernel.
+//  k_moe_down: blocks of one token: waves split the picks, each pick's dots of a pass of output rows
+//    land in LDS and are combined in pick order (deterministic), with down's bias.
 //
-// Decode is bound by memory latency rather than bandwidth (a layer reads ~7 MB), so both kernels
-// issue all their weight loads before anything that waits: the IQ grid copy into LDS and the
-// barrier come after the loads are in flight.
+// and, for one token of the shapes it is built for, in one (k_moe_decode).
 #include <stddef.h>
 
 #include <mutex>
@@ -60,146 +58,238 @@ __device__ __forceinline__ typename F::Raw load_rc(const uint8_t *mat, int64_t r
     else return F::load(mat + r * rb, sb);
 }
 
-template <class Fmt, int LPR, int NX, int PER, int ROWS>
+// Routes token t in one wave (wave_route, by the count of experts) and gives lane j < K its pick's
+// slot: the expert itself, or the bank's table entry (an absent expert reads slot 0), ~0u past the bank.
+__device__ __forceinline__ void route_token(const MoeArgs &a, int t, uint32_t &rid, float &rw, uint32_t &slot, bool &absent) {
+    const float *logits = a.logits + (int64_t)t * a.E;
+    if (a.E <= 256) wave_route<4>(logits, a.E, a.K, a.norm, &rid, &rw);
+    else if (a.E <= 512) wave_route<8>(logits, a.E, a.K, a.norm, &rid, &rw);
+    else wave_route<16>(logits, a.E, a.K, a.norm, &rid, &rw);
+    slot = 0xFFFFFFFFu;
+    absent = false;
+    if ((int)(threadIdx.x & 63) < a.K) {
+        slot = a.table ? a.table[rid] : rid;
+        absent = slot == CW_NO_SLOT;
+        if (absent) slot = 0;
+        if (slot >= (uint32_t)a.n_slots) slot = 0xFFFFFFFFu;
+    }
+}
+
+template <class Fmt, int LPR, int NX>
+struct GateUpShape {
+    static constexpr int RAW = (int)(sizeof(typename Fmt::Raw) / 4);         // registers of a sub-block's raw bytes
+    static constexpr int ROWS = LPR == 64 && NX == 1 && RAW <= 8 ? 2 : 1;    // rows of an item, per 64/LPR
+    static constexpr bool AHEAD = 2 * ROWS * NX * RAW <= 40;                 // room for a second item's bytes
+};
+// blockIdx.y = token t; its blocks' waves stride over the token's items (pick, ROWS * 64/LPR rows
+// of gate and up). Wave 0 routes the token once per block, the token's x stays in registers and the
+// lattice tables in LDS for every item of the block, and an item's weight bytes are requested
+// (unconditionally, from clamped rows and sub-blocks) while the item before it is computed. What
+// bounds it: the dots' VALU work (config 3's shape at 8 tokens: 134M weights of about two
+// instructions each) and the memory round trips of a block's start. With a block per (pick, 8 rows),
+// each wave of it routing the token and reading x for two rows, and down in blocks of 4 rows that
+// each filled the tables, the layer took 77.6 us at 8 tokens and takes 38.8 now; 25.6
+// and 18.9 at 2 tokens; MXFP4 at 2,880 x 2,880, top-4, 8 tokens: 319 and 164 (same output bits but
+// for the rows with three sub-blocks per lane).
+template <class Fmt, int LPR, int NX>
 __global__ __launch_bounds__(256) void k_moe_gateup(const MoeArgs a) {
     __shared__ __align__(16) uint8_t lds[Fmt::LDS_BYTES > 0 ? Fmt::LDS_BYTES : 16];
-    constexpr int RPW = 64 / LPR;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = blockDim.x >> 6;
+    __shared__ uint32_t pick_slot[32], pick_e[32];
+    using S = GateUpShape<Fmt, LPR, NX>;
+    constexpr int RPW = 64 / LPR, ROWS = S::ROWS;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int sub = lane % LPR, rsub = lane / LPR;
-    const int p = blockIdx.y, t = p / a.K, j = p - t * a.K;
-
-    uint32_t rid;
-    float rw;
-    wave_route<PER>(a.logits + (int64_t)t * a.E, a.E, a.K, a.norm, &rid, &rw);
-    const uint32_t expert = __shfl(rid, j);
-    uint32_t slot = a.table ? a.table[expert] : expert;
-    const bool absent = slot == CW_NO_SLOT;
-    if (absent) slot = 0;
-    const bool bad = slot >= (uint32_t)a.n_slots;
-    const float wj = __shfl(rw, j);
-    if (blockIdx.x == 0 && wave == 0 && lane == 0) {
-        a.ids[p] = expert;
-        a.w[p] = wj;
-        a.slots[p] = bad ? 0xFFFFFFFFu : slot;
-        if (absent && a.missing) atomicAdd(a.missing, 1u);
-    }
-
-    // weight loads for ROWS passes, in flight before anything waits
-    const uint8_t *bg = a.wg + (int64_t)(bad ? 0 : slot) * a.sg;
-    const uint8_t *bu = a.wu + (int64_t)(bad ? 0 : slot) * a.su;
-    const int nsb = a.H / 32;
-    const int r_first = (blockIdx.x * nwaves + wave) * RPW * ROWS + rsub;
-    typename Fmt::Raw rg[ROWS][NX], ru[ROWS][NX];
-#pragma unroll
-    for (int q = 0; q < ROWS; q++) {
-        const int r = r_first + q * RPW;
-#pragma unroll
-        for (int i = 0; i < NX; i++) {
-            const int sb = sub + i * LPR;
-            if (r < a.I && sb < nsb) {
-                rg[q][i] = load_rc<Fmt>(bg, r, a.rbg, sb);
-                ru[q][i] = load_rc<Fmt>(bu, r, a.rbg, sb);
+    const int t = blockIdx.y, K = a.K, nsb = a.H / 32;
+    if (wave == 0) {
+        uint32_t rid, slot;
+        float rw;
+        bool absent;
+        route_token(a, t, rid, rw, slot, absent);
+        if (lane < K) {
+            pick_slot[lane] = slot;
+            pick_e[lane] = rid;
+            if (blockIdx.x == 0) {
+                a.ids[t * K + lane] = rid;
+                a.w[t * K + lane] = rw;
+                a.slots[t * K + lane] = slot;
+                if (absent && a.missing) atomicAdd(a.missing, 1u);
             }
         }
     }
-    float xr[NX][32];
+    float xr[NX][32], xs[NX][2];
     load_xs<NX>(xr, a.x + (int64_t)t * a.H, sub, LPR, nsb);
     Fmt::fill_lds(lds, threadIdx.x, blockDim.x);
-    if (Fmt::LDS_BYTES > 0) __syncthreads();
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NX; i++) half_sums(xr[i], xs[i]);
 
-    const int P = a.P;
+    const int ngrp = (a.I + RPW * ROWS - 1) / (RPW * ROWS), stride = gridDim.x * 4;
+    struct Item {
+        typename Fmt::Raw g[ROWS][NX], u[ROWS][NX];
+    };
+    auto fetch = [&](int j, int grp, Item &it) __attribute__((always_inline)) {
+        const uint32_t slot = __builtin_amdgcn_readfirstlane(pick_slot[j]), sl = slot == 0xFFFFFFFFu ? 0 : slot;
+        const uint8_t *bg = a.wg + (int64_t)sl * a.sg, *bu = a.wu + (int64_t)sl * a.su;
 #pragma unroll
-    for (int q = 0; q < ROWS; q++) {
-        const int r = r_first + q * RPW;
-        float g = 0.f, u = 0.f;
+        for (int q = 0; q < ROWS; q++) {
+            const int r = min((grp * ROWS + q) * RPW + rsub, a.I - 1);
 #pragma unroll
-        for (int i = 0; i < NX; i++) {
-            const int sb = sub + i * LPR;
-            if (r < a.I && sb < nsb) {
-                g += Fmt::dot(rg[q][i], lds, xr[i]);
-                u += Fmt::dot(ru[q][i], lds, xr[i]);
+            for (int i = 0; i < NX; i++) {
+                const int sb = min(sub + i * LPR, nsb - 1);
+                it.g[q][i] = load_rc<Fmt>(bg, r, a.rbg, sb);
+                it.u[q][i] = load_rc<Fmt>(bu, r, a.rbg, sb);
             }
         }
-        g = group_sum<LPR>(g);
-        u = group_sum<LPR>(u);
-        if (sub == 0 && r < a.I) {
+    };
+    // the item's pick and row group, moved on by `stride` items without a division
+    int j = 0, grp = blockIdx.x * 4 + wave;
+    while (j < K && grp >= ngrp) { grp -= ngrp; j++; }
+    Item cur, nxt;
+    if (S::AHEAD && j < K) fetch(j, grp, cur);
+    while (j < K) {
+        int jn = j, gn = grp + stride;
+        while (jn < K && gn >= ngrp) { gn -= ngrp; jn++; }
+        if constexpr (S::AHEAD) fetch(jn < K ? jn : j, jn < K ? gn : grp, nxt);  // past the last item: the same one again, unused
+        else fetch(j, grp, cur);
+        float g[ROWS], u[ROWS];
+#pragma unroll
+        for (int q = 0; q < ROWS; q++) {
+            g[q] = 0.f;
+            u[q] = 0.f;
+#pragma unroll
+            for (int i = 0; i < NX; i++) {
+                const float dg = dot_xs<Fmt>(cur.g[q][i], lds, xr[i], xs[i]), du = dot_xs<Fmt>(cur.u[q][i], lds, xr[i], xs[i]);
+                const bool in = sub + i * LPR < nsb;  // (a clamped sub-block's scale may be infinite: not x = 0 alone)
+                g[q] += in ? dg : 0.f;
+                u[q] += in ? du : 0.f;
+            }
+            g[q] = group_sum<LPR>(g[q]);
+            u[q] = group_sum<LPR>(u[q]);
+        }
+        // the activation once, with row q of each group in the group's lane q
+        float gv = g[0], uv = u[0];
+#pragma unroll
+        for (int q = 1; q < ROWS; q++) {
+            gv = sub == q ? g[q] : gv;
+            uv = sub == q ? u[q] : uv;
+        }
+        const int r = (grp * ROWS + sub) * RPW + rsub;
+        if (sub < ROWS && r < a.I) {
             float o;
             if (a.act == CW_ACT_SILU) {
-                o = g / (1.0f + expf(-g)) * u;
+                o = gv / (1.0f + expf(-gv)) * uv;
             } else {
-                if (a.bg) g += a.bg[(int64_t)expert * a.I + r];
-                if (a.bu) u += a.bu[(int64_t)expert * a.I + r];
-                g = fminf(g, a.limit);
-                u = fminf(fmaxf(u, -a.limit), a.limit);
-                o = (u + 1.0f) * (g * (1.0f / (1.0f + expf(-(g * a.alpha)))));
+                const int64_t e = pick_e[j];
+                if (a.bg) gv += a.bg[e * a.I + r];
+                if (a.bu) uv += a.bu[e * a.I + r];
+                gv = fminf(gv, a.limit);
+                uv = fminf(fmaxf(uv, -a.limit), a.limit);
+                o = (uv + 1.0f) * (gv * (1.0f / (1.0f + expf(-(gv * a.alpha)))));
             }
-            a.h[(int64_t)p * P + r] = bad ? __int_as_float(0x7fc00000) : o;
+            a.h[(int64_t)(t * K + j) * a.P + r] = pick_slot[j] == 0xFFFFFFFFu ? __int_as_float(0x7fc00000) : o;
         }
+        if constexpr (S::AHEAD) cur = nxt;
+        j = jn;
+        grp = gn;
     }
-    // zero padding of the hidden row up to the width down reads
-    for (int c = a.I + blockIdx.x * blockDim.x + threadIdx.x; c < P; c += gridDim.x * blockDim.x)
-        a.h[(int64_t)p * P + c] = 0.f;
+    // zero padding of the hidden rows up to the width down reads
+    const int padw = a.P - a.I;
+    for (int c = blockIdx.x * 256 + threadIdx.x; c < K * padw; c += gridDim.x * 256)
+        a.h[(int64_t)(t * K + c / padw) * a.P + a.I + c % padw] = 0.f;
 }
 
 // ------------------------------------------------------------------------------ down + combine
 
-// tile = 64/LPR rows: one pass of every wave per pick
+// blockIdx.y = token; a block of W waves takes passes of U * 64/LPR output rows, wave w the picks
+// w, w + W, ... (PPW of them), whose hidden rows it holds in registers for all of the block's passes
+// (XREG; where they do not fit, each dot reads its slice again). A pass's weight bytes are requested
+// together; the picks' dots meet in LDS (two buffers: one barrier per pass) and are combined in pick
+// order, so the result does not depend on the split.
 template <class Fmt, int LPR, int NX, int PPW>
-__global__ __launch_bounds__(256) void k_moe_down(const MoeArgs a) {
+struct DownShape {
+    static constexpr bool XREG = PPW * NX <= 4;
+    static constexpr int RAW = PPW * NX * (int)(sizeof(typename Fmt::Raw) / 4);  // registers of a row group's raw bytes
+    static constexpr int U = RAW <= 12 ? 4 : RAW <= 24 ? 2 : 1;
+    static constexpr int RPP = U * (64 / LPR);  // rows of a pass
+};
+template <class Fmt, int LPR, int NX, int PPW>
+__global__ __launch_bounds__(512) void k_moe_down(const MoeArgs a) {
+    using S = DownShape<Fmt, LPR, NX, PPW>;
+    constexpr int RPW = 64 / LPR, U = S::U, RPP = S::RPP;
     __shared__ __align__(16) uint8_t lds[Fmt::LDS_BYTES > 0 ? Fmt::LDS_BYTES : 16];
-    __shared__ float part[32 * (64 / LPR)];
-    constexpr int RPW = 64 / LPR;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = blockDim.x >> 6;
+    __shared__ float part[2][32 * RPP];
+    __shared__ float pick_w[32];
+    __shared__ uint32_t pick_e[32];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
     const int sub = lane % LPR, rsub = lane / LPR;
-    const int t = blockIdx.y;
-    const int r = blockIdx.x * RPW + rsub;
-    const int nsb = a.P / 32;
+    const int t = blockIdx.y, K = a.K, nsb = a.P / 32;
 
-    // PPW picks per wave: j = wave + q * nwaves
-    typename Fmt::Raw raw[PPW][NX];
-    float xr[PPW][NX][32];
+    const uint8_t *base[PPW];
     bool bad[PPW];
+    float xr[S::XREG ? PPW : 1][NX][32], xs[S::XREG ? PPW : 1][NX][2];
 #pragma unroll
     for (int q = 0; q < PPW; q++) {
-        const int j = wave + q * nwaves;
-        bad[q] = true;
-        if (j < a.K) {
-            const uint32_t slot = a.slots[t * a.K + j];
-            bad[q] = slot >= (uint32_t)a.n_slots;
-            const uint8_t *base = a.wd + (int64_t)(bad[q] ? 0 : slot) * a.sd;
-#pragma unroll
-            for (int i = 0; i < NX; i++) {
-                const int sb = sub + i * LPR;
-                if (r < a.H && sb < nsb) raw[q][i] = load_rc<Fmt>(base, r, a.rbd, sb);
-            }
-            load_xs<NX>(xr[q], a.h + (int64_t)(t * a.K + j) * a.P, sub, LPR, nsb);
-        }
+        const int j = min(wave + q * nw, K - 1);  // past the picks: the last one again, unused
+        const uint32_t slot = __builtin_amdgcn_readfirstlane(a.slots[t * K + j]);
+        bad[q] = slot >= (uint32_t)a.n_slots;
+        base[q] = a.wd + (int64_t)(bad[q] ? 0 : slot) * a.sd;
+        if constexpr (S::XREG) load_xs<NX>(xr[q], a.h + (int64_t)(t * K + j) * a.P, sub, LPR, nsb);
+    }
+    if ((int)threadIdx.x < K) {
+        pick_w[threadIdx.x] = a.w[t * K + threadIdx.x];
+        pick_e[threadIdx.x] = a.ids[t * K + threadIdx.x];
     }
     Fmt::fill_lds(lds, threadIdx.x, blockDim.x);
-    if (Fmt::LDS_BYTES > 0) __syncthreads();
+    if constexpr (S::XREG) {
 #pragma unroll
-    for (int q = 0; q < PPW; q++) {
-        const int j = wave + q * nwaves;
-        if (j >= a.K) break;  // uniform across the wave
-        float d = 0.f;
+        for (int q = 0; q < PPW; q++)
 #pragma unroll
-        for (int i = 0; i < NX; i++) {
-            const int sb = sub + i * LPR;
-            if (r < a.H && sb < nsb) d += Fmt::dot(raw[q][i], lds, xr[q][i]);
-        }
-        d = group_sum<LPR>(d);
-        if (sub == 0) part[j * RPW + rsub] = bad[q] ? __int_as_float(0x7fc00000) : d;
+            for (int i = 0; i < NX; i++) half_sums(xr[q][i], xs[q][i]);
     }
     __syncthreads();
-    if (threadIdx.x < RPW) {
-        const int rr = blockIdx.x * RPW + threadIdx.x;
-        if (rr < a.H) {
+    int buf = 0;
+    for (int r0 = blockIdx.x * RPP; r0 < a.H; r0 += gridDim.x * RPP, buf ^= 1) {
+        typename Fmt::Raw raw[PPW][U][NX];
+#pragma unroll
+        for (int q = 0; q < PPW; q++)
+#pragma unroll
+            for (int v = 0; v < U; v++)
+#pragma unroll
+                for (int i = 0; i < NX; i++)
+                    raw[q][v][i] = load_rc<Fmt>(base[q], min(r0 + v * RPW + rsub, a.H - 1), a.rbd, min(sub + i * LPR, nsb - 1));
+#pragma unroll
+        for (int q = 0; q < PPW; q++) {
+            const int j = wave + q * nw;
+            if (j >= K) break;  // uniform across the wave
+#pragma unroll
+            for (int v = 0; v < U; v++) {
+                float d = 0.f;
+#pragma unroll
+                for (int i = 0; i < NX; i++) {
+                    float e;
+                    if constexpr (S::XREG) {
+                        e = dot_xs<Fmt>(raw[q][v][i], lds, xr[q][i], xs[q][i]);
+                    } else {
+                        float x1[32];
+                        const float4 *src = (const float4 *)(a.h + (int64_t)(t * K + j) * a.P + 32 * min(sub + i * LPR, nsb - 1));
+#pragma unroll
+                        for (int c = 0; c < 8; c++) *(float4 *)(x1 + 4 * c) = src[c];
+                        e = Fmt::dot(raw[q][v][i], lds, x1);
+                    }
+                    d += sub + i * LPR < nsb ? e : 0.f;
+                }
+                d = group_sum<LPR>(d);
+                if (sub == 0) part[buf][j * RPP + v * RPW + rsub] = bad[q] ? __int_as_float(0x7fc00000) : d;
+            }
+        }
+        __syncthreads();
+        const int rr = r0 + threadIdx.x;
+        if (threadIdx.x < RPP && rr < a.H) {
             float acc = 0.f;
-            for (int j = 0; j < a.K; j++) {
-                const int pick = t * a.K + j;
-                float d = part[j * RPW + threadIdx.x];
-                if (a.bd) d += a.bd[(int64_t)a.ids[pick] * a.H + rr];
-                acc += a.w[pick] * d;
+            for (int j = 0; j < K; j++) {
+                float d = part[buf][j * RPP + threadIdx.x];
+                if (a.bd) d += a.bd[(int64_t)pick_e[j] * a.H + rr];
+                acc += pick_w[j] * d;
             }
             a.out[(int64_t)t * a.H + rr] = acc;
         }
@@ -985,45 +1075,57 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : 1) void k_moe_decode(const Mo
 
 // ------------------------------------------------------------------------------ dispatch
 
-static int lpr_for(int nsb) {
-    int l = 8;
-    while (l < nsb && l < 64) l <<= 1;
-    return l;
+// blocks (of all tokens) that keep the device's CUs busy without more block starts than needed:
+// about 16 waves per CU
+static int blocks_per_token(int waves, int T, int want) {
+    const int all = 256 * 16 / waves, per = (all + T - 1) / T;
+    return want < per ? want : per;
 }
 
 template <class Fmt, int LPR, int NX>
-static int gateup_per(const MoeArgs &a, int T, hipStream_t s) {
-    constexpr int RPW = 64 / LPR;
-    constexpr int ROWS = LPR == 64 ? 2 : 1;
-    const int rows_per_block = 4 * RPW * ROWS;
-    dim3 grid((a.I + rows_per_block - 1) / rows_per_block, T * a.K);
-    if (a.E <= 256) hipLaunchKernelGGL((k_moe_gateup<Fmt, LPR, NX, 4, ROWS>), grid, dim3(256), 0, s, a);
-    else if (a.E <= 512) hipLaunchKernelGGL((k_moe_gateup<Fmt, LPR, NX, 8, ROWS>), grid, dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((k_moe_gateup<Fmt, LPR, NX, 16, ROWS>), grid, dim3(256), 0, s, a);
+static int gateup_launch(const MoeArgs &a, int T, hipStream_t s) {
+    constexpr int RPI = 64 / LPR * GateUpShape<Fmt, LPR, NX>::ROWS;
+    const int64_t items = (int64_t)a.K * ((a.I + RPI - 1) / RPI);
+    const dim3 grid((unsigned)blocks_per_token(4, T, (int)((items + 3) / 4)), (unsigned)T);
+    hipLaunchKernelGGL((k_moe_gateup<Fmt, LPR, NX>), grid, dim3(256), 0, s, a);
     return check_launch("k_moe_gateup");
 }
 
-template <class Fmt, int LPR, int NX>
-static int down_per(const MoeArgs &a, int T, hipStream_t s) {
-    constexpr int RPW = 64 / LPR;
-    dim3 grid((a.H + RPW - 1) / RPW, T);
-    const int ppw = (a.K + 3) / 4;
-    if (ppw == 1) hipLaunchKernelGGL((k_moe_down<Fmt, LPR, NX, 1>), grid, dim3(256), 0, s, a);
-    else if (ppw == 2) hipLaunchKernelGGL((k_moe_down<Fmt, LPR, NX, 2>), grid, dim3(256), 0, s, a);
-    else if (ppw <= 4) hipLaunchKernelGGL((k_moe_down<Fmt, LPR, NX, 4>), grid, dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((k_moe_down<Fmt, LPR, NX, 8>), grid, dim3(256), 0, s, a);
+template <class Fmt, int LPR, int NX, int PPW>
+static int down_launch(const MoeArgs &a, int T, hipStream_t s) {
+    constexpr int RPP = DownShape<Fmt, LPR, NX, PPW>::RPP;
+    const int waves = (a.K + PPW - 1) / PPW;  // at most 8
+    const dim3 grid((unsigned)blocks_per_token(waves, T, (a.H + RPP - 1) / RPP), (unsigned)T);
+    hipLaunchKernelGGL((k_moe_down<Fmt, LPR, NX, PPW>), grid, dim3(64 * waves), 0, s, a);
     return check_launch("k_moe_down");
 }
 
+template <class Fmt, bool DOWN, int LPR, int NX>
+static int token_launch(const MoeArgs &a, int T, hipStream_t s) {
+    if constexpr (!DOWN) {
+        return gateup_launch<Fmt, LPR, NX>(a, T, s);
+    } else {
+        if (a.K <= 8) return down_launch<Fmt, LPR, NX, 1>(a, T, s);
+        if (a.K <= 16) return down_launch<Fmt, LPR, NX, 2>(a, T, s);
+        return down_launch<Fmt, LPR, NX, 4>(a, T, s);
+    }
+}
+
+// Lanes per row (LPR) and sub-blocks per lane (NX) of a row of nsb sub-blocks: a wave's work is
+// LPR * NX sub-block slots per row, so 33..48 and 65..96 sub-blocks (1,056..1,536 and 2,080..3,072
+// weights) take 3 per lane at 16 and 32 lanes: 48 and 96 slots instead of 64 and 128.
 template <class Fmt, bool DOWN>
 static int by_shape(const MoeArgs &a, int T, hipStream_t s) {
     const int nsb = (DOWN ? a.P : a.H) / 32;
-    const int lpr = lpr_for(nsb);
-    const int nx = (nsb + lpr - 1) / lpr;
-#define CW_CASE(L, X) \
-    if (lpr == L && nx == X) return DOWN ? down_per<Fmt, L, X>(a, T, s) : gateup_per<Fmt, L, X>(a, T, s);
-    CW_CASE(8, 1) CW_CASE(16, 1) CW_CASE(32, 1) CW_CASE(64, 1) CW_CASE(64, 2) CW_CASE(64, 3) CW_CASE(64, 4)
-#undef CW_CASE
+    if (nsb <= 8) return token_launch<Fmt, DOWN, 8, 1>(a, T, s);
+    if (nsb <= 16) return token_launch<Fmt, DOWN, 16, 1>(a, T, s);
+    if (nsb <= 32) return token_launch<Fmt, DOWN, 32, 1>(a, T, s);
+    if (nsb <= 48) return token_launch<Fmt, DOWN, 16, 3>(a, T, s);
+    if (nsb <= 64) return token_launch<Fmt, DOWN, 64, 1>(a, T, s);
+    if (nsb <= 96) return token_launch<Fmt, DOWN, 32, 3>(a, T, s);
+    if (nsb <= 128) return token_launch<Fmt, DOWN, 64, 2>(a, T, s);
+    if (nsb <= 192) return token_launch<Fmt, DOWN, 64, 3>(a, T, s);
+    if (nsb <= 256) return token_launch<Fmt, DOWN, 64, 4>(a, T, s);
     return set_error(CW_ENOTSUP, "moe: rows of %d weights exceed %d", nsb * 32, 64 * 4 * 32);
 }
 
