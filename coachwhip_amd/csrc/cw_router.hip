@@ -7,9 +7,9 @@
 //
 //  - A few tokens (decode): one wave per expert row; lanes stride the row in 4-element pieces,
 //    each piece of W read once and used for every token; a DPP wave sum per token.
-//  - Many tokens (prefill): a 64-expert x 64-token tile per block, K in chunks of 32 staged in
-//    LDS (k-major, so a thread's 4 experts and 4 tokens are one 16-byte read each), 4 x 4
-//    outputs per thread.
+//  - Many tokens (prefill): 32 x 32 tiles on the f32 matrix instruction, K in chunks through LDS.
+#include <atomic>
+
 #include "cw_common.h"
 #include "cw_router.h"
 #include "cw_wave.h"
@@ -58,48 +58,57 @@ __global__ __launch_bounds__(256) void k_router_rows(const WT *w, const float *b
     }
 }
 
+// 32 tokens x 32 experts per block, one 16 x 16 tile per wave on v_mfma_f32_16x16x4_f32, whose sum
+// is the chain fma(a_k, b_k, acc) over ascending k, one rounding each (subnormals kept): the logits
+// are those of a scalar loop over k, bit for bit, and do not depend on the tile. K goes through LDS in
+// chunks of 256, the next chunk's loads in flight during this one's 64 MFMAs; rows 260 floats apart
+// put the 64 lanes of a fragment read on distinct banks. What bounds it is that chain (32 cycles per
+// 4 weights, 6.8 us for 2,048); 64 x 64 tiles on the VALU (10 blocks for 301 tokens x 128 experts, a
+// round trip to memory per 32 of K) took 122 us where this takes 19.6 (1,500 x 256: 147 and 41.6).
+constexpr int RT = 32, RKC = 256, RLD = RKC + 4;
 template <class WT>
 __global__ __launch_bounds__(256) void k_router_tiles(const WT *w, const float *bias, const float *x, int E, int h, int T,
                                                       float *logits) {
-    constexpr int TE = 64, TTK = 64, KC = 32, PAD = 4;
-    __shared__ __align__(16) float Ws[KC][TE + PAD], Xs[KC][TTK + PAD];
-    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-    const int e0 = blockIdx.x * TE, t0 = blockIdx.y * TTK;
-    float acc[4][4] = {};
-    // loader: thread tid copies 4 consecutive k of row (tid >> 3) and (tid >> 3) + 32, piece tid & 7
-    const int lr = tid >> 3, lk = 4 * (tid & 7);
-    for (int kc = 0; kc < h; kc += KC) {
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    extern __shared__ __align__(16) float rs[];  // two buffers of RT token rows, then RT expert rows
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, grp = lane >> 4;
+    const int e0 = blockIdx.x * RT, t0 = blockIdx.y * RT;
+    // wave w copies rows w, w + 4, ... of the chunk, lane l 4 floats from 4 l (rows and columns past
+    // the matrices: a clamped address, zeros stored)
+    float4 v[2 * RT / 4];
+    auto fetch = [&](int kc) __attribute__((always_inline)) {
+        const int k = kc + 4 * lane, kk = k < h ? k : h - 4;
 #pragma unroll
-        for (int half = 0; half < 2; half++) {
-            const int r = lr + 32 * half;
-            const int e = e0 + r, t = t0 + r, k = kc + lk;
-            const float4 a = e < E && k < h ? load4<WT>(w + (int64_t)e * h + k) : make_float4(0.f, 0.f, 0.f, 0.f);
-            const float4 b = t < T && k < h ? *(const float4 *)(x + (int64_t)t * h + k) : make_float4(0.f, 0.f, 0.f, 0.f);
-            Ws[lk][r] = a.x; Ws[lk + 1][r] = a.y; Ws[lk + 2][r] = a.z; Ws[lk + 3][r] = a.w;
-            Xs[lk][r] = b.x; Xs[lk + 1][r] = b.y; Xs[lk + 2][r] = b.z; Xs[lk + 3][r] = b.w;
+        for (int i = 0; i < 2 * RT / 4; i++) {
+            const int r = 4 * i + wave;
+            if (r < RT) v[i] = *(const float4 *)(x + (int64_t)min(t0 + r, T - 1) * h + kk);
+            else v[i] = load4<WT>(w + (int64_t)min(e0 + r - RT, E - 1) * h + kk);
         }
-        __syncthreads();
-#pragma unroll 8
-        for (int k = 0; k < KC; k++) {
-            const float4 a = *(const float4 *)&Ws[k][4 * tx];
-            const float4 b = *(const float4 *)&Xs[k][4 * ty];
-            const float av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w};
+        if (k >= h) {
 #pragma unroll
-            for (int i = 0; i < 4; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) acc[i][j] = fmaf(av[i], bv[j], acc[i][j]);
+            for (int i = 0; i < 2 * RT / 4; i++) v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
         }
-        __syncthreads();
+    };
+    fetch(0);
+    const int tr = 16 * (wave & 1), er = 16 * (wave >> 1);
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int kc = 0, b = 0; kc < h; kc += RKC, b ^= 1) {
+        float *buf = rs + b * 2 * RT * RLD;
+#pragma unroll
+        for (int i = 0; i < 2 * RT / 4; i++) *(float4 *)(buf + (4 * i + wave) * RLD + 4 * lane) = v[i];
+        __syncthreads();  // (the other buffer is refilled only after the next one)
+        if (kc + RKC < h) fetch(kc + RKC);
+        const float *xa = buf + (tr + l16) * RLD + grp, *wb = buf + (RT + er + l16) * RLD + grp;
+#pragma unroll
+        for (int j = 0; j < RKC / 4; j++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[4 * j], wb[4 * j], acc, 0, 0, 0);
     }
+    const int e = e0 + er + l16;
+    if (e >= E) return;
+    const float be = bias ? bias[e] : 0.f;
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int t = t0 + 4 * ty + j;
-        if (t >= T) break;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int e = e0 + 4 * tx + i;
-            if (e < E) logits[(int64_t)t * E + e] = acc[i][j] + (bias ? bias[e] : 0.f);
-        }
+    for (int i = 0; i < 4; i++) {
+        const int t = t0 + tr + 4 * grp + i;
+        if (t < T) logits[(int64_t)t * E + e] = acc[i] + be;
     }
 }
 
@@ -113,7 +122,18 @@ static int launch(const void *w, const float *bias, const float *x, int E, int h
         CW_ROWS(1) CW_ROWS(2) CW_ROWS(4) CW_ROWS(8)
 #undef CW_ROWS
     }
-    hipLaunchKernelGGL((k_router_tiles<WT>), dim3((E + 63) / 64, (T + 63) / 64), dim3(256), 0, s, wt, bias, x, E, h, T, logits);
+    // dynamic LDS above 64 KB, opted into once per device
+    constexpr int MAX_DEVICES = 64;
+    constexpr size_t lds = 2 * 2 * RT * RLD * sizeof(float);
+    static std::atomic<bool> lds_set[MAX_DEVICES];
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES) dev = 0;
+    if (!lds_set[dev].load(std::memory_order_acquire)) {
+        if (hipFuncSetAttribute((const void *)k_router_tiles<WT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+            return set_error(CW_EHIP, "router: cannot reserve %zu bytes of LDS", lds);
+        lds_set[dev].store(true, std::memory_order_release);
+    }
+    hipLaunchKernelGGL((k_router_tiles<WT>), dim3((E + RT - 1) / RT, (T + RT - 1) / RT), dim3(256), lds, s, wt, bias, x, E, h, T, logits);
     return check_launch("k_router_tiles");
 }
 
