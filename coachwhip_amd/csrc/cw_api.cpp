@@ -94,10 +94,24 @@ static bool qmatmul_mfma(int dtype, int64_t k, int64_t m) {
            (dtype == CW_Q8_0 || dtype == CW_MXFP4 || k % 256 == 0);
 }
 
+// Q5_K and Q6_K: whether m rows run as the f32-accurate GEMM (activations as two fp16 terms; matrices
+// below its 4 GiB). Graph-replayed on MI355X, a matvec takes about 2.2 us + 0.17 us per row and million
+// weights (Q6_K 4096 x 4096: 16.8 us at 4 rows, 22.5 at 6), the pack and the GEMM about 9.5 us + 0.4 us
+// per million weights (17.5 and 17.6): equal at (m - 2.4) n k = 43 million. Measured either side: 1024 x
+// 2048 at 16 rows 11.0 (matvec) and 12.9, 16384 x 2048 at 4 rows 27.8 and 20.3. Without a workspace the
+// call stays on the matvec. CWMOE_MM_MIN_ROWS (rows) overrides.
+static bool qmatmul_split(int dtype, int64_t n, int64_t k, int64_t m) {
+    if ((dtype != CW_Q5_K && dtype != CW_Q6_K) || m >= (1 << 24) || k % 256 || k > 8192 || n <= 0 || n >= (1ll << 31) ||
+        n * (k / 256 * cw_type_size(dtype)) >= (1ll << 32))
+        return false;
+    if (const char *e = getenv("CWMOE_MM_MIN_ROWS")) return m >= atoll(e);
+    return m > 2 && (5 * m - 12) * n * k >= 215000000ll;
+}
+
 size_t cw_qmatmul_workspace_size(int dtype, int64_t n, int64_t k, int64_t m) {
-    (void)n;
-    if (!is_weight_type(dtype) || k <= 0 || m <= 0 || !qmatmul_mfma(dtype, k, m)) return 0;
-    return cw::mfma_dense_workspace(dtype, m, n, k);
+    if (!is_weight_type(dtype) || k <= 0 || m <= 0) return 0;
+    if (qmatmul_split(dtype, n, k, m)) return n > 0 ? cw::split_dense_workspace(dtype, m, n, k) : 0;
+    return qmatmul_mfma(dtype, k, m) ? cw::mfma_dense_workspace(dtype, m, n, k) : 0;
 }
 
 int cw_qmatmul(int dtype, const void *w, int64_t n, int64_t k, const float *x, int64_t m, float *y, void *ws,
@@ -114,6 +128,9 @@ int cw_qmatmul(int dtype, const void *w, int64_t n, int64_t k, const float *x, i
     if (qmatmul_mfma(dtype, k, m))
         return cw::mfma_dense(dtype, (const uint8_t *)w, k / bs * cw_type_size(dtype), (int)n, (int)k, x, (int)m, y, ws,
                               ws_bytes, (hipStream_t)stream);
+    if (qmatmul_split(dtype, n, k, m) && ws && ws_bytes >= cw::split_dense_workspace(dtype, m, n, k))
+        return cw::split_dense(dtype, (const uint8_t *)w, k / bs * cw_type_size(dtype), (int)n, (int)k, x, (int)m, y, ws, ws_bytes,
+                               (hipStream_t)stream);
     GemvArgs a = {};
     a.w0 = (const uint8_t *)w;
     a.row_bytes = k / bs * cw_type_size(dtype);

@@ -72,6 +72,16 @@ struct PackExtra {
     int n_zero;
 };
 
+// launch arithmetic shared by the GEMMs: the current device (below MAX_DEVICES), its persistent blocks
+// (per_cu per CU, a multiple of 8, the XCD count), M-tiles per run of work items, work items, and the
+// split count of a dense matmul (rpb weight rows per item, stages of kst K-steps)
+constexpr int MAX_DEVICES = 64;
+int current_device();
+int64_t resident_blocks(int per_cu = 1);
+int run_of_tiles(int64_t tiles);
+int64_t gemm_items(int64_t tiles, int rpb, int64_t n);
+int dense_splits(int rpb, int kst, int per_cu, int64_t m, int64_t n, int64_t k, int &split_st);
+
 bool mfma_supported(int dtype);
 // formats whose MFMA fragments take each 32-wide K step in a permuted order (MXFP4: a byte's two
 // nibbles side by side); their activations are packed with pack_rows_f16(..., perm = true)
@@ -94,6 +104,18 @@ int mfma_dense(int dtype, const uint8_t *w, int64_t row_bytes, int n, int k, con
 // pick with slots[t*K+j] >= n_slots contributes NaN (it has no row)
 int combine_picks(const float *dn, const float *w, const float *bias, const uint32_t *ids, const uint32_t *slots, int n_slots,
                   int T, int K, int H, float *out, hipStream_t s);
+
+// The same GEMMs at f32 accuracy (cw_mfma_split.hip): activations as two fp16 terms, exact weight codes.
+// Rows of split_row halves, packed for the weights' format.
+bool split_supported(int dtype);
+int split_row(int dtype, int64_t k);
+int pack_rows_split(int dtype, const float *x, int rows, int k, int ldx, uint16_t *a16, float *ascale, hipStream_t s,
+                    const PackExtra *extra = nullptr);
+int split_gateup(int dtype, const MfArgs &a, int tiles_max, hipStream_t s);
+int split_down(int dtype, const MfArgs &a, int tiles_max, hipStream_t s);
+size_t split_dense_workspace(int dtype, int64_t m, int64_t n, int64_t k);
+int split_dense(int dtype, const uint8_t *w, int64_t row_bytes, int n, int k, const float *x, int m, float *y, void *ws, size_t ws_bytes,
+                hipStream_t s);
 
 // MXFP4 grouped GEMMs on the block-scaled MFMA (cw_mxfp4.hip): the weights as stored (E2M1 codes
 // and E8M0 block scales), the activations as three FP6 terms with E8M0 scales per 32 values.

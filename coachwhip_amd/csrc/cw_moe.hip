@@ -102,7 +102,7 @@ static int route(const float *logits, int T, int E, int K, int norm, uint32_t *i
 struct MoeLayout {
     size_t state, ids, w, slots, g, u, h, total;
     // grouped (MFMA) path
-    bool grouped;
+    bool grouped, split;  // split: at f32 accuracy (activations as two fp16 terms)
     size_t pile_pick, pile_tok, tiles, n_tiles, x16, xscale, h16, hscale, dn;
 };
 
@@ -131,6 +131,28 @@ static uint32_t decode_polls() {
 static bool grouped_path(const cw_moe_desc *d, int T) {
     return T >= prefill_min_tokens() && d->dtype[0] == d->dtype[1] && mfma_supported(d->dtype[0]) &&
            mfma_supported(d->dtype[2]) && (d->slot_table ? d->n_slots : d->n_experts) <= 1024;
+}
+
+// Layers with a Q5_K or Q6_K matrix have no fp16 GEMM: they run as grouped GEMMs at f32 accuracy (their
+// per-pick matvecs keep f32 activations), where the other formats of the layer can too and every matrix is
+// below the GEMM's 4 GiB, once that is faster. The matvecs read an expert's matrices once per pick
+// (measured about 0.235 us per million weights, + 10 us), the GEMMs once per distinct expert (about 0.245
+// us per million, + 45 us for their launches and rounds), so the GEMMs win where the picks beyond the
+// distinct experts, E (1 - (1 - K / E)^T) on average, come to 150 million weights or more; 230 here, since
+// near the line the matvecs spread better. Measured (matvec / GEMM): Q4_K + Q6_K, 128 experts, top-8, 768
+// x 2048: 16 tokens 136 / 144, 24 tokens 229 / 161; 256 experts of 512: 16 tokens 88 / 128, 24 tokens 150
+// / 149. CWMOE_PREFILL_MIN_TOKENS (tokens) overrides.
+static bool split_path(const cw_moe_desc *d, int T) {
+    if (grouped_path(d, T) || d->dtype[0] != d->dtype[1] || !split_supported(d->dtype[0]) ||
+        !split_supported(d->dtype[2]) || (d->slot_table ? d->n_slots : d->n_experts) > 1024)
+        return false;
+    const int P = d->pad > d->inter ? d->pad : d->inter;
+    const int64_t gu = (int64_t)d->inter * (d->hidden / cw_block_size(d->dtype[0])) * cw_type_size(d->dtype[0]);
+    const int64_t dn = (int64_t)d->hidden * (P / cw_block_size(d->dtype[2])) * cw_type_size(d->dtype[2]);
+    if (gu >= ((int64_t)1 << 32) || dn >= ((int64_t)1 << 32) || (int64_t)T * d->top_k >= (1 << 28)) return false;
+    if (getenv("CWMOE_PREFILL_MIN_TOKENS")) return T >= prefill_min_tokens();
+    const double K = d->top_k, E = std::max<double>(d->slot_table ? d->n_slots : d->n_experts, K), distinct = E * (1 - pow(1 - K / E, T));
+    return (T * K - distinct) * d->hidden * (2.0 * d->inter + P) >= 230e6;
 }
 
 static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -168,7 +190,8 @@ static int check_desc(const cw_moe_desc *d, int T) {
     return CW_OK;
 }
 
-static MoeLayout layout(const cw_moe_desc *d, int T) {
+// allow_split: off for callers whose scratch holds the matvecs' layout but not the split GEMMs'
+static MoeLayout layout(const cw_moe_desc *d, int T, bool allow_split = true) {
     const size_t TK = (size_t)T * d->top_k;
     const int P = d->pad > d->inter ? d->pad : d->inter;
     MoeLayout L;
@@ -183,7 +206,8 @@ static MoeLayout layout(const cw_moe_desc *d, int T) {
     L.g = off; off = align256(off + (split ? TK * d->inter * 4 : 0));
     L.u = off; off = align256(off + (split ? TK * d->inter * 4 : 0));
     L.h = off; off = align256(off + TK * (size_t)P * 4);
-    L.grouped = grouped_path(d, T);
+    L.split = allow_split && split_path(d, T);
+    L.grouped = L.split || grouped_path(d, T);
     if (L.grouped) {
         const int n_slots = d->slot_table ? d->n_slots : d->n_experts;
         L.pile_pick = off; off = align256(off + TK * 4);
@@ -192,9 +216,10 @@ static MoeLayout layout(const cw_moe_desc *d, int T) {
         L.n_tiles = off; off = align256(off + 4);
         // fp16 rows, or for MXFP4 on the scaled MFMA the rows packed as FP6 terms
         const bool gx = mxfp4_scaled_for(d->dtype[0], d->hidden), dx = mxfp4_scaled_for(d->dtype[2], P);
-        L.x16 = off; off = align256(off + (gx ? fp6_rows_bytes(T, d->hidden) : (size_t)T * d->hidden * 2));
+        const size_t xrow = L.split ? split_row(d->dtype[0], d->hidden) : d->hidden, hrow = L.split ? split_row(d->dtype[2], P) : P;
+        L.x16 = off; off = align256(off + (gx ? fp6_rows_bytes(T, d->hidden) : (size_t)T * xrow * 2));
         L.xscale = off; off = align256(off + (size_t)T * 4);
-        L.h16 = off; off = align256(off + (dx ? fp6_rows_bytes((int64_t)TK, P) : TK * (size_t)P * 2));
+        L.h16 = off; off = align256(off + (dx ? fp6_rows_bytes((int64_t)TK, P) : TK * hrow * 2));
         L.hscale = off; off = align256(off + TK * 4);
         L.dn = off; off = align256(off + TK * (size_t)d->hidden * 4);
     }
@@ -221,6 +246,7 @@ static int moe_grouped(const cw_moe_desc *d, const MoeArgs &a, const MoeLayout &
     // MXFP4 matrices run on the block-scaled MFMA (activations as FP6 terms), the others on fp16 MFMA
     const bool gx = mxfp4_scaled_for(d->dtype[0], a.H), dx = mxfp4_scaled_for(d->dtype[2], P);
     if (gx) rc = pack_rows_fp6(a.x, T, a.H, a.H, (uint8_t *)x16, s);
+    else if (L.split) rc = pack_rows_split(d->dtype[0], a.x, T, a.H, a.H, x16, xscale, s);
     else rc = pack_rows_f16(a.x, T, a.H, a.H, x16, xscale, s, nullptr, mfma_k_permuted(d->dtype[0]));
     if (rc) return rc;
     // gate/up and down both on the scaled MFMA: gate/up packs the hidden rows itself
@@ -238,7 +264,7 @@ static int moe_grouped(const cw_moe_desc *d, const MoeArgs &a, const MoeLayout &
     g.k = a.H;
     g.a16 = x16;
     g.ascale = xscale;
-    g.lda = a.H;
+    g.lda = L.split ? split_row(d->dtype[0], a.H) : a.H;
     g.rows = pile_tok;
     g.tiles = tiles;
     g.n_tiles = n_tiles;
@@ -263,12 +289,15 @@ static int moe_grouped(const cw_moe_desc *d, const MoeArgs &a, const MoeLayout &
             g.hp_blocks = (int)(g.hp_row / 304 * 4);
         }
         rc = mxfp4_gateup(g, tmax, s);
+    } else if (L.split) {
+        rc = split_gateup(d->dtype[0], g, tmax, s);
     } else {
         rc = mfma_gateup(d->dtype[0], g, tmax, s);
     }
     if (rc) return rc;
     if (fuse_h) rc = CW_OK;
     else if (dx) rc = pack_rows_fp6(a.h, TK, P, P, (uint8_t *)h16, s);
+    else if (L.split) rc = pack_rows_split(d->dtype[2], a.h, TK, P, P, h16, hscale, s);
     else rc = pack_rows_f16(a.h, TK, P, P, h16, hscale, s, nullptr, mfma_k_permuted(d->dtype[2]));
     if (rc) return rc;
 
@@ -280,7 +309,7 @@ static int moe_grouped(const cw_moe_desc *d, const MoeArgs &a, const MoeLayout &
     dn.k = P;
     dn.a16 = h16;
     dn.ascale = hscale;
-    dn.lda = P;
+    dn.lda = L.split ? split_row(d->dtype[2], P) : P;
     dn.rows = nullptr;
     dn.tiles = tiles;
     dn.n_tiles = n_tiles;
@@ -293,6 +322,8 @@ static int moe_grouped(const cw_moe_desc *d, const MoeArgs &a, const MoeLayout &
         dn.ap_row = (int64_t)fp6_rows_bytes(1, P);
         dn.ap_rows = TK;
         rc = mxfp4_down(dn, tmax, s);
+    } else if (L.split) {
+        rc = split_down(d->dtype[2], dn, tmax, s);
     } else {
         rc = mfma_down(d->dtype[2], dn, tmax, s);
     }
@@ -306,7 +337,8 @@ static int moe_layer(const cw_moe_desc *d, const float *x, const float *logits, 
     if (rc) return rc;
     if (T == 0) return CW_OK;
     CW_REQUIRE(x && logits && out, "moe: null x, logits or out");
-    const MoeLayout L = layout(d, T);
+    MoeLayout L = layout(d, T);
+    if (L.split && ws_bytes < L.total) L = layout(d, T, false);
     CW_REQUIRE(ws && ws_bytes >= L.total, "moe: workspace of %zu bytes, %zu needed", ws_bytes, L.total);
     uint8_t *base = (uint8_t *)ws;
     const int K = d->top_k, P = d->pad > d->inter ? d->pad : d->inter;
@@ -684,7 +716,7 @@ int cw_moe_layer_noalloc(const cw_moe_desc *desc, const float *x, const float *l
     int rc = check_desc(desc, T);
     if (rc) return rc;
     if (T == 0) return CW_OK;
-    const size_t need = layout(desc, T).total;
+    const size_t need = layout(desc, T, false).total;  // (the split GEMMs where their layout fits too)
     if (need > NOALLOC_SCRATCH_BYTES)
         return set_error(CW_EINVAL, "moe noalloc: %d tokens need %zu bytes of scratch, above the %zu the library holds", T, need,
                          NOALLOC_SCRATCH_BYTES);

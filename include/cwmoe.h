@@ -102,7 +102,9 @@ int cw_dequantize(int dtype, const void *blocks, int64_t n_elems, float *out, cw
  * vendor/candle-metal-kernels/src/kernels/quantized.rs:32-43, 198-213).
  * From 2 rows of x (Q4_K) or 8 rows (the other formats) the product runs as an MFMA GEMM on
  * fp16-rounded activations (rel-L2 about 3e-4 against f64) and needs the workspace; below that
- * it is one f32 matvec per row. ws may be NULL when cw_qmatmul_workspace_size returns 0. */
+ * it is one f32 matvec per row. Q5_K and Q6_K keep f32 accuracy at every m: a matvec per row, or, for
+ * as many rows as pay for it, a GEMM on the activations as two fp16 terms (it needs the workspace; a
+ * call without one takes the matvecs). ws may be NULL when cw_qmatmul_workspace_size returns 0. */
 size_t cw_qmatmul_workspace_size(int dtype, int64_t n, int64_t k, int64_t m);
 int cw_qmatmul(int dtype, const void *w, int64_t n, int64_t k, const float *x, int64_t m,
                float *y, void *ws, size_t ws_bytes, cw_stream_t stream);
@@ -251,7 +253,8 @@ int cw_moe_layer(const cw_moe_desc *desc, const float *x, const float *logits, i
  * larger is refused with CW_EINVAL (config 3's shape fits about 90 tokens). The call allocates
  * nothing. Every call on a device shares that device's array: calls that overlap in time on one
  * device (on different streams, or from different threads) race and must not be made. Outputs
- * equal cw_moe_layer's bit for bit (the same kernels). */
+ * equal cw_moe_layer's bit for bit (the same kernels; a layer with Q5_K or Q6_K matrices whose GEMMs'
+ * workspace does not fit the array takes the per-pick matvecs instead: equal to f32 accuracy). */
 #define CW_MOE_NOALLOC_BYTES ((size_t)8 << 20)
 int cw_moe_layer_noalloc(const cw_moe_desc *desc, const float *x, const float *logits, int T,
                          float *out, uint32_t *ids_out, float *w_out, uint32_t *missing,
