@@ -83,16 +83,20 @@ int64_t gemm_items(int64_t tiles, int rpb, int64_t n);
 int dense_splits(int rpb, int kst, int per_cu, int64_t m, int64_t n, int64_t k, int &split_st);
 
 bool mfma_supported(int dtype);
-// formats whose MFMA fragments take each 32-wide K step in a permuted order (MXFP4: a byte's two
-// nibbles side by side); their activations are packed with pack_rows_f16(..., perm = true)
-inline bool mfma_k_permuted(int dtype) { return dtype == CW_MXFP4; }
+// The K order of a format's MFMA fragments, in which its activations are packed: natural; MXFP4's (a
+// byte's two nibbles side by side); or by octets of lane-owned sub-blocks within each super-block (the
+// formats with SB in cw_gmm_dev.h).
+enum { K_NATURAL = 0, K_PAIRS = 1, K_OCTETS = 2 };
+inline int k_order(int dtype) {
+    return dtype == CW_MXFP4 ? K_PAIRS : dtype == CW_Q8_0 || dtype == CW_IQ4_XS ? K_NATURAL : K_OCTETS;
+}
 // one block: expert piles of the (slot) picks, and the tile list
 int mfma_piles(const uint32_t *slots, const uint32_t *ids, int TK, int K, int n_slots, int *pile_pick, int *pile_tok, MfTile *tiles,
                int *n_tiles, hipStream_t s);
 int max_tiles(int TK, int n_slots);
-// rows x k f32 -> fp16 rows (ld = k) with per-row power-of-two scales
+// rows x k f32 -> fp16 rows (ld = k, K order as given) with per-row power-of-two scales
 int pack_rows_f16(const float *x, int rows, int k, int ldx, uint16_t *a16, float *ascale, hipStream_t s,
-                  const PackExtra *extra = nullptr, bool perm = false);
+                  const PackExtra *extra = nullptr, int order = K_NATURAL);
 int fill_zero(float *p, int64_t n, hipStream_t s);
 int mfma_gateup(int dtype, const MfArgs &a, int tiles_max, hipStream_t s);
 int mfma_down(int dtype, const MfArgs &a, int tiles_max, hipStream_t s);

@@ -312,7 +312,7 @@ __global__ __launch_bounds__(1024, 4) void k_gmm(const MfArgs a) {
                     for (int q = 0; q < NB; q++) {
                         // the accumulators move onto the new scale at the start of the K-steps (only
                         // the tile's pick blocks); a zero scale keeps the old one (its codes do not count)
-                        const float d = MF::scale(win[m][q]);
+                        const float d = stg[m][q].d;
                         zero[m][q] = d == 0.f;
                         ratio[m][q] = d != 0.f ? rs[m][q] * __builtin_amdgcn_rcpf(d) : 1.f;
                         rs[m][q] = d != 0.f ? d : rs[m][q];
@@ -647,7 +647,7 @@ __global__ __launch_bounds__(1024) void k_piles(const uint32_t *slots, const uin
 // One wave per row, the row held in registers (NV float4 per lane, k <= 256*NV): scale =
 // 2^(15 - e) with max|x| in [2^(e-1), 2^e) keeps the row's largest value in [2^14, 2^15) of
 // fp16; ascale receives 1/scale.
-template <int NV, bool PERM>
+template <int NV, int ORDER>
 __global__ __launch_bounds__(256) void k_pack_f16(const float *x, int rows, int k, int ldx, uint16_t *a16, float *ascale,
                                                   PackExtra e) {
     pack_extra(e);
@@ -657,7 +657,7 @@ __global__ __launch_bounds__(256) void k_pack_f16(const float *x, int rows, int 
     float4 v[NV];
     float m = 0.f;
     // loads from clamped addresses (all in flight at once), the values past the row zeroed after
-    if constexpr (PERM) {
+    if constexpr (ORDER == K_PAIRS) {
         // positions c..c+3 of a 32-wide step take its elements 2t, 2t+16, 2t+1, 2t+17 (t = (c % 32) / 4)
 #pragma unroll
         for (int i = 0; i < NV; i++) {
@@ -682,9 +682,12 @@ __global__ __launch_bounds__(256) void k_pack_f16(const float *x, int rows, int 
     if (m > 0.f && m < INFINITY) { frexpf(m, &ex); ex = 15 - ex; }
     const float sc = ldexpf(1.0f, ex);
     uint16_t *o = a16 + (int64_t)row * k;
+    // K_OCTETS: the lane's 4 values are half (lane & 1) of octet l = (lane >> 1) & 3 of sub-block 4j + g =
+    // lane >> 3: positions 32 (4j + l) + 8g
+    const int c0 = ORDER == K_OCTETS ? 128 * (lane >> 5) + 32 * ((lane >> 1) & 3) + 8 * ((lane >> 3) & 3) + 4 * (lane & 1) : 4 * lane;
 #pragma unroll
     for (int i = 0; i < NV; i++) {
-        const int c = 4 * lane + 256 * i;
+        const int c = c0 + 256 * i;
         if (c < k) {
             const uint32_t lo = __builtin_bit_cast(uint16_t, (_Float16)(v[i].x * sc)) | ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(v[i].y * sc)) << 16);
             const uint32_t hi = __builtin_bit_cast(uint16_t, (_Float16)(v[i].z * sc)) | ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(v[i].w * sc)) << 16);
@@ -759,17 +762,19 @@ int mfma_piles(const uint32_t *slots, const uint32_t *ids, int TK, int K, int n_
 }
 
 int pack_rows_f16(const float *x, int rows, int k, int ldx, uint16_t *a16, float *ascale, hipStream_t s,
-                  const PackExtra *extra, bool perm) {
+                  const PackExtra *extra, int order) {
     if (rows == 0) return CW_OK;
     if (k % 4 || ldx % 4) return set_error(CW_ENOTSUP, "pack: row of %d (stride %d) is not whole float4s", k, ldx);
-    if (perm && k % 32) return set_error(CW_ENOTSUP, "pack: a permuted row of %d is not whole 32-wide steps", k);
+    if (order != K_NATURAL && k % (order == K_OCTETS ? 256 : 32))
+        return set_error(CW_ENOTSUP, "pack: a permuted row of %d is not whole steps", k);
     const dim3 grid((rows + 3) / 4);
     const int nv = (k + 255) / 256;
     const PackExtra e = extra ? *extra : PackExtra{};
 #define CW_PACK(N) \
     if (nv <= N) { \
-        if (perm) hipLaunchKernelGGL((k_pack_f16<N, true>), grid, dim3(256), 0, s, x, rows, k, ldx, a16, ascale, e); \
-        else hipLaunchKernelGGL((k_pack_f16<N, false>), grid, dim3(256), 0, s, x, rows, k, ldx, a16, ascale, e); \
+        if (order == K_PAIRS) hipLaunchKernelGGL((k_pack_f16<N, K_PAIRS>), grid, dim3(256), 0, s, x, rows, k, ldx, a16, ascale, e); \
+        else if (order == K_OCTETS) hipLaunchKernelGGL((k_pack_f16<N, K_OCTETS>), grid, dim3(256), 0, s, x, rows, k, ldx, a16, ascale, e); \
+        else hipLaunchKernelGGL((k_pack_f16<N, K_NATURAL>), grid, dim3(256), 0, s, x, rows, k, ldx, a16, ascale, e); \
         return check_launch("k_pack_f16"); \
     }
     CW_PACK(2) CW_PACK(4) CW_PACK(8) CW_PACK(12) CW_PACK(16) CW_PACK(32)
@@ -1026,7 +1031,7 @@ __global__ __launch_bounds__(64 * W) void k_skinny_q4k(const uint8_t *w, int64_t
 static int dense_skinny_q4k(const uint8_t *w, int64_t row_bytes, int n, int k, const float *x, int m, float *y, uint16_t *x16,
                             float *xs, hipStream_t s) {
     int rc;
-    if ((rc = pack_rows_f16(x, m, k, k, x16, xs, s, nullptr, false))) return rc;
+    if ((rc = pack_rows_f16(x, m, k, k, x16, xs, s, nullptr, K_NATURAL))) return rc;
     const int nsb = k / 256, waves = (nsb + SKINNY_SB - 1) / SKINNY_SB;
     const dim3 grid((unsigned)((n + 15) / 16));
     if (waves <= 1) hipLaunchKernelGGL(k_skinny_q4k<1>, grid, dim3(64), 0, s, w, row_bytes, n, k, x16, xs, m, y);
@@ -1061,7 +1066,7 @@ int mfma_dense(int dtype, const uint8_t *w, int64_t row_bytes, int n, int k, con
     // one launch packs x, writes the tile list and zeroes the split counters
     const PackExtra extra = {tiles, n_tiles, m, cnt, S > 1 ? (int)dense_items(dtype, m, n) : 0};
     int rc;
-    if ((rc = pack_rows_f16(x, m, k, k, x16, xs, s, &extra, mfma_k_permuted(dtype)))) return rc;
+    if ((rc = pack_rows_f16(x, m, k, k, x16, xs, s, &extra, k_order(dtype)))) return rc;
     MfArgs a = {};
     a.w0 = w;
     a.s0 = 0;

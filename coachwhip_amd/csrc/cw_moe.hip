@@ -247,7 +247,7 @@ static int moe_grouped(const cw_moe_desc *d, const MoeArgs &a, const MoeLayout &
     const bool gx = mxfp4_scaled_for(d->dtype[0], a.H), dx = mxfp4_scaled_for(d->dtype[2], P);
     if (gx) rc = pack_rows_fp6(a.x, T, a.H, a.H, (uint8_t *)x16, s);
     else if (L.split) rc = pack_rows_split(d->dtype[0], a.x, T, a.H, a.H, x16, xscale, s);
-    else rc = pack_rows_f16(a.x, T, a.H, a.H, x16, xscale, s, nullptr, mfma_k_permuted(d->dtype[0]));
+    else rc = pack_rows_f16(a.x, T, a.H, a.H, x16, xscale, s, nullptr, k_order(d->dtype[0]));
     if (rc) return rc;
     // gate/up and down both on the scaled MFMA: gate/up packs the hidden rows itself
     const bool fuse_h = gx && dx;
@@ -298,7 +298,7 @@ static int moe_grouped(const cw_moe_desc *d, const MoeArgs &a, const MoeLayout &
     if (fuse_h) rc = CW_OK;
     else if (dx) rc = pack_rows_fp6(a.h, TK, P, P, (uint8_t *)h16, s);
     else if (L.split) rc = pack_rows_split(d->dtype[2], a.h, TK, P, P, h16, hscale, s);
-    else rc = pack_rows_f16(a.h, TK, P, P, h16, hscale, s, nullptr, mfma_k_permuted(d->dtype[2]));
+    else rc = pack_rows_f16(a.h, TK, P, P, h16, hscale, s, nullptr, k_order(d->dtype[2]));
     if (rc) return rc;
 
     MfArgs dn = {};
@@ -597,7 +597,7 @@ int cw_matmul_id_grouped(int dtype, int64_t n, int64_t k, int64_t n_slots, int64
     if ((rc = mfma_piles(ids, nullptr, TK, K, (int)n_slots, pile_pick, pile_tok, tiles, n_tiles, s))) return rc;
     const bool gx = mxfp4_scaled_for(dtype, k);
     if (gx) rc = pack_rows_fp6(x, xpp ? TK : T, (int)k, (int)k, (uint8_t *)x16, s);
-    else rc = pack_rows_f16(x, xpp ? TK : T, (int)k, (int)k, x16, xscale, s, nullptr, mfma_k_permuted(dtype));
+    else rc = pack_rows_f16(x, xpp ? TK : T, (int)k, (int)k, x16, xscale, s, nullptr, k_order(dtype));
     if (rc) return rc;
     MfArgs a = {};
     a.w0 = (const uint8_t *)bank;
