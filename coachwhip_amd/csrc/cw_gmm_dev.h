@@ -545,29 +545,28 @@ template <int V> struct Ic { static constexpr int value = V; };
 
 __device__ __forceinline__ f16x8 as_f16x8(uint4 v) { return __builtin_bit_cast(f16x8, v); }
 
-// 16 bytes from global memory to LDS without passing through registers: lane l of the wave
-// writes lds_base + 16*l (lds_base is the same for the whole wave).
-// ASM: issued as inline asm instead of through __builtin_amdgcn_global_load_lds. The compiler
-// counts the builtin as an LDS store that any later LDS read at a dynamic address (a table
-// lookup) may alias, and puts an s_waitcnt vmcnt(0) before that read, so every prefetch is
-// waited for right after it is issued. The kernel orders these loads itself: an explicit
-// s_waitcnt on the issuing wave, then a barrier, before any wave reads the bytes, and a barrier
-// between the last read of a buffer and the loads that overwrite it. Loads return in order, so
-// the compiler's own vmcnt waits stay correct with these in flight (they only wait longer: a
-// register spill's reload then waits for the prefetches before it, which is why the formats
-// that spill keep the builtin).
-template <bool ASM>
-__device__ __forceinline__ void dma16(const void *g, uint8_t *lds_base) {
-    if constexpr (ASM) {
-        const uint32_t m = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t *)lds_base);
-        // M0 (the LDS base of the load) is reserved to the compiler, which may keep a value in it:
-        // saved and restored around the load
-        uint32_t keep;
-        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b32 m0, %0"
-                     : "=&s"(keep) : "v"(g), "s"(m) : "memory");
-    } else {
-        __builtin_amdgcn_global_load_lds(g, (__attribute__((address_space(3))) void *)lds_base, 16, 0, 0);
-    }
+// Direct global-to-LDS loads, without passing through registers: lane l of the wave writes 16 (or 4)
+// bytes at an LDS address, the same for the whole wave, + 16 l (4 l). Issued as inline asm instead of
+// through __builtin_amdgcn_global_load_lds: the compiler counts the builtin as an LDS store that any later
+// LDS read at a dynamic address (a table lookup) may alias, and puts an s_waitcnt vmcnt(0) before that
+// read, so every prefetch is waited for right after it is issued. A kernel orders these loads itself: an
+// explicit s_waitcnt on the issuing wave, then a barrier, before any wave reads the bytes, and a barrier
+// between the last read of a buffer and the loads that overwrite it. Loads return in order, so the
+// compiler's own vmcnt waits stay correct with these in flight (they only wait longer: a register spill's
+// reload then waits for the prefetches before it).
+__device__ __forceinline__ uint32_t lds_addr(const void *p) {
+    return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t *)p);
+}
+// base: wave-uniform; off: the lane's 32-bit offset
+__device__ __forceinline__ void dma16_s(const uint8_t *base, uint32_t off, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "s"(lds) : "memory", "m0");
+}
+// g: the lane's address
+__device__ __forceinline__ void dma16(const void *g, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(g), "s"(lds) : "memory", "m0");
+}
+__device__ __forceinline__ void dma4(const void *g, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" : : "v"(g), "s"(lds) : "memory", "m0");
 }
 
 // The end of a split-K work item (MODE 2), its partial rows stored: the last block to get here sums them.

@@ -1,9 +1,8 @@
 // Grouped expert GEMMs on MFMA (gfx950, v_mfma_f32_16x16x32_f16) for the MoE layer's prefill.
 //
 // Picks are grouped by the slot they read (mfma_piles); a tile is up to MF_MT = 80 picks of one
-// slot (5 MFMA blocks of 16) by RPB weight rows per matrix. A block has 16 waves for gate/up
-// (8 on gate, 8 on up) and 8 for down and dense matmuls; each wave owns 16 weight rows and every
-// pick block of the tile.
+// slot (5 MFMA blocks of 16) by RPB weight rows per matrix. A block has 8 waves (for gate/up, 4 on
+// gate and 4 on up); each wave owns 16 weight rows and every pick block of the tile.
 //
 // Exactness: a weight is (f16 super-block scale) x (small integer code). The codes go through
 // MFMA as fp16 integers, which they represent exactly: IQ2_XXS / IQ2_S codes (2s+1)*grid*sign
@@ -36,34 +35,48 @@ struct GmShape {
     static constexpr int LDS_MAX = 160 * 1024;
     static constexpr int NM = MODE == 0 ? 2 : 1;
     static constexpr int NB = 1;
-    // PF: K-step table lookups and activation fragments read one step ahead (two register sets).
-    // ADMA: the stage loads issued as inline asm (dma16). Both for every format but MXFP4 (equal or
-    // slower with either).
-    static constexpr bool FAST = !std::is_same<MF, MMXFP4>::value;
-    static constexpr bool PF = FAST, ADMA = FAST;
-    // K-steps per activation buffer and buffers per stage. Q4_K's down and dense instances take 2:
-    // the halved buffers make room for a second window buffer beside two blocks per CU.
-    static constexpr int KA = std::is_same<MF, MQ4_K>::value && MODE != 0 ? 2 : 4, HPS = MF::KST / KA;
-    static constexpr int A_HALF = KA * MF_MB * 64 * 16, A_BYTES = 2 * A_HALF;  // two activation buffers
-    static constexpr int META_BYTES = MF_MT * 8;                     // scale and pick of each row of the tile
-    static constexpr int FIXED = ((MF::LDS + 15) & ~15) + A_BYTES + META_BYTES;
-    // Gate/up: 16 waves (one block per CU), where their windows fit beside the tables. Down and
-    // dense: 8 waves, two blocks per CU where the LDS allows, so one block's item start and end
-    // (with a short K: down's is 512) overlap the other's K-steps. A wave works on one matrix:
-    // the first WPM waves on gate, the others on up (MODE 0), which keeps its registers to one
-    // accumulator set.
-    static constexpr int NW = MODE == 0 && FIXED + 16 * 16 * Win<MF>::BYTES <= LDS_MAX ? 16 : 8, NT = 64 * NW;
+    // PF: K-step table lookups and activation fragments read one step ahead (two register sets),
+    // for every format but MXFP4 (equal or slower).
+    static constexpr bool PF = !std::is_same<MF, MMXFP4>::value;
+    // Blocks of 8 waves, two per CU, so one block's item start and end and its barriers' waits overlap
+    // the other's K-steps. A wave works on one matrix (MODE 0: the first WPM waves on gate, the others on
+    // up), which keeps its registers to one accumulator set.
+    static constexpr int NW = 8, NT = 64 * NW, PER_CU = 2;
     static constexpr int WPM = NW / NM;                              // waves per matrix
     static constexpr int RPW = 16 * NB, RPB = WPM * RPW;
     static constexpr int W_BYTES = NM * RPB * Win<MF>::BYTES;       // one stage of weight windows
-    // 8-wave blocks run two per CU where two fit. Two window buffers are taken where they fit
-    // beside the rest (without costing the second block): the weights of stage st+1 then load
-    // while stage st computes.
-    static constexpr int BASE_BYTES = FIXED + W_BYTES;
-    static constexpr int PER_CU = NW == 8 && 2 * BASE_BYTES <= LDS_MAX ? 2 : 1;  // resident blocks per CU
-    static constexpr bool WDB = PER_CU * (BASE_BYTES + W_BYTES) <= LDS_MAX;
-    static constexpr size_t lds_bytes() { return BASE_BYTES + (WDB ? W_BYTES : 0); }
-    static_assert(BASE_BYTES <= LDS_MAX, "the GEMM's LDS does not fit");
+    static constexpr int META_BYTES = 2 * 128 * 4;                   // scale and pick of each row of the tile, by whole waves
+    // The stage's activations load in HPS parts of KA K-steps, into a ring of as many parts of the tile's
+    // pick blocks as the space of two full tiles holds; the windows into a ring of NWB stages. KA = 4
+    // where three stages of windows fit beside it, else 2.
+    static constexpr int a_bytes(int ka) { return 2 * ka * MF_MB * 64 * 16; }
+    static constexpr int room(int ka) { return LDS_MAX / PER_CU - ((MF::LDS + 15) & ~15) - a_bytes(ka) - META_BYTES; }
+    static constexpr int KA = room(4) >= 3 * W_BYTES ? 4 : 2, HPS = MF::KST / KA;
+    static constexpr int NWB = room(KA) >= 3 * W_BYTES ? 3 : 2;
+    static constexpr int A_BYTES = a_bytes(KA);
+    // parts of the activation ring for MBS pick blocks: a part is requested NA - 1 parts ahead, and never
+    // before the windows of its stage
+    static constexpr int na(int mbs) {
+        const int n = 2 * MF_MB / mbs, m = 1 + (NWB - 1) * HPS;
+        return n < m ? (n < 5 ? n : 5) : (m < 5 ? m : 5);
+    }
+    // Loads that may still be in flight when part hp of a stage starts: what its wave has requested after
+    // the part's activations and, for the stage's first part, after the stage's windows (loads return in
+    // order). ntw: a wave's window loads per stage; ka: its activation loads per part (0 for the waves
+    // that load none).
+    static constexpr int in_flight(int hp, int NA, int ntw, int ka) {
+        int n = ka * (NA - 2);
+        for (int i = 1; i <= NA - 1; i++) n += (hp - i) % HPS == 0 ? ntw : 0;  // stage starts among the parts since
+        if (hp == 0) {
+            const int parts = (NWB - 1) * HPS - 1 < NA - 1 ? (NWB - 1) * HPS - 1 : NA - 1;
+            const int w = ka * parts + ntw * (NWB - 2);
+            if (w < n) n = w;
+        }
+        return n < 63 ? n : 63;
+    }
+    static constexpr int BASE_BYTES = ((MF::LDS + 15) & ~15) + A_BYTES + META_BYTES + NWB * W_BYTES;
+    static constexpr size_t lds_bytes() { return BASE_BYTES; }
+    static_assert(PER_CU * BASE_BYTES <= LDS_MAX, "the GEMM's LDS does not fit");
     static_assert(MODE != 0 || MF_MT * RPB * 4 <= A_BYTES, "the gate/up exchange does not fit the activation buffers");
 };
 
@@ -76,9 +89,18 @@ struct GmShape {
 // into LDS with direct global-to-LDS loads: activations in MFMA fragment order ([K-step][pick
 // block][lane] x 16 bytes, so every fragment read is one conflict-free ds_read_b128), weights as
 // one window of whole 16-byte pieces per row (each load instruction covers 1 KB of consecutive
-// pieces, instead of a few bytes from each of 16 rows). Latency is hidden by the second block
-// on the CU. A piece is loaded only when it holds a byte of the row's stage; an aligned 16-byte
+// pieces, instead of a few bytes from each of 16 rows). A piece is loaded only when it holds a byte of the row's stage; an aligned 16-byte
 // piece cannot cross a page boundary, so its other bytes are mapped memory too.
+//
+// What bounds it: instructions. A wave's stage was about 300 VALU and 250 scalar instructions around 8
+// fragments (half of them load addresses worked out in 64 bits, LDS addresses cast through a generic
+// pointer, and M0 saved around every load); loads from a uniform base with 32-bit lane offsets, LDS
+// addresses kept as such and rows that start on 16 bytes (Q4_K) taken as one constant make it about 230
+// and 100. Longer prefetches alone (the rings below, before that) changed nothing. Two 8-wave blocks per
+// CU for gate/up instead of one of 16 gave 8 % at 64 tokens. Layers, before and after all of it: 256 IQ2
+// experts, top-8, 2048 x 512, 32 tokens 122 -> 106 us, 64 tokens 157 -> 137, 1,500 tokens 239 -> 230; 128
+// Q4_K experts, 768 x 2048, 256 tokens 155 -> 145; 64 IQ4_XS experts, 16 tokens 121 -> 91; dense Q8_0 4096 x
+// 4096, 512 rows 83 -> 65.
 //
 // Scales: the accumulator of a weight row carries a running scale. When a new scale unit starts
 // (an IQ super-block, or an MXFP4 stage), the accumulator is multiplied by old/new scale and the
@@ -95,9 +117,9 @@ __global__ __launch_bounds__(1024, 4) void k_gmm(const MfArgs a) {
     __shared__ int split_last;  // split-K: this block finished its work item's last split
     uint8_t *tab = smem;
     uint8_t *As = smem + ((MF::LDS + 15) & ~15);
-    uint8_t *Ws = As + S::A_BYTES;  // window buffer(s): stage st uses Ws + (WDB ? st & 1 : 0) * W_BYTES
-    float *meta_sa = (float *)(Ws + (S::WDB ? 2 : 1) * S::W_BYTES);
-    int *meta_pick = (int *)(meta_sa + MF_MT);
+    uint8_t *Ws = As + S::A_BYTES;
+    float *meta_sa = (float *)(Ws + S::NWB * S::W_BYTES);
+    int *meta_pick = (int *)(meta_sa + 128);
     const int n_nb = (a.n + S::RPB - 1) / S::RPB;
     // blocks go to the 8 XCDs round-robin; item b of each run of R*n_nb (R = run_tiles) takes
     // M-tile R*run + b%R and N-block b/R. With R = 8 an M-tile's N-blocks share an XCD (and its
@@ -121,20 +143,21 @@ __global__ __launch_bounds__(1024, 4) void k_gmm(const MfArgs a) {
         const MfTile tile = a.tiles[mt];
         const int mbs = (tile.m + 15) >> 4;
 
-        // the epilogue's activation scale and pick index of tile row tid, fetched now and put in LDS
-        // with the first stage
-        float my_sa = 0.f;
-        int my_pick = 0;
-        if (tid < tile.m) {
-            const int pos = tile.pos0 + tid;
-            my_sa = a.ascale[a.rows ? a.rows[pos] : pos];
-            my_pick = a.pile_pick ? a.pile_pick[pos] : pos;
-        }
+        // The epilogue's activation scale and pick index of each tile row, by the first two waves straight
+        // into LDS (rows past the tile's last: that one's, unused), published by the first part's barrier.
+        const int mpos = tile.pos0 + min(tid, tile.m - 1);
+        const int mrow = a.rows && wave < 2 ? a.rows[mpos] : mpos;
 
         // the activation row this lane copies: pick block `wave`, row l16, k-group grp
         const bool stager = wave < mbs;
         const int apos = tile.pos0 + min(16 * wave + l16, tile.m - 1);
         const uint16_t *asrc = a.a16 + (int64_t)(a.rows ? a.rows[apos] : apos) * a.lda + 8 * grp;
+
+        if (wave < 2) {
+            dma4(a.ascale + mrow, lds_addr(meta_sa) + 256 * wave);
+            if (a.pile_pick) dma4(a.pile_pick + mpos, lds_addr(meta_pick) + 256 * wave);
+            else meta_pick[tid] = mpos;
+        }
 
         // Row r of the block is row nblk*RPB + r % RPB of matrix r / RPB (rows past n read row 0).
         // Addresses are the block's matrix base (uniform) plus 32-bit offsets (a matrix is under
@@ -168,167 +191,166 @@ __global__ __launch_bounds__(1024, 4) void k_gmm(const MfArgs a) {
                 }
             }
 
-        // The weight windows of stage st_w into buffer wbuf: every wave issues exactly NTW loads
-        // (waves past the last piece repeat the first ones, writing the same bytes to the same place,
-        // and pieces past a row's last one re-load that one into a slot nothing reads), so the
-        // stage's wait can leave exactly the next stage's loads in flight. RPB*PCS is a multiple of
-        // 64: a wave's pieces lie in one matrix and the matrix base stays scalar.
+        // The weight windows of stage st_w into buffer wbuf (an LDS address): every wave issues exactly NTW
+        // loads (waves past the last piece repeat the first ones, writing the same bytes to the same
+        // place, and pieces past a row's last one re-load that one into a slot nothing reads), so a
+        // stage's wait can leave exactly the loads after it in flight. RPB*PCS is a multiple of 64: a
+        // wave's pieces lie in one matrix and the matrix base stays scalar. A piece's row offset and its
+        // place in the row's window are the same in every stage, so they are worked out once per tile
+        // (the division by the window's piece count and the row's 32-bit multiply), from the 16-byte
+        // boundary at or below the matrix base: wp_off the row's first byte, wp_p the piece.
         constexpr int NP = S::NM * S::RPB * W::PCS, NTW = (NP + S::NT - 1) / S::NT;
-        // A piece's row offset and its place in the row's window are the same in every stage: for
-        // the formats with registers to spare (S::FAST) they are worked out once per tile (the
-        // division by the window's piece count and the row's 32-bit multiply were most of the
-        // stage's address arithmetic), the others recompute them per stage.
+        static_assert(S::RPB * W::PCS % 64 == 0, "a wave's pieces lie in one matrix");
+        const uint32_t b0 = (uint32_t)(uintptr_t)wb0 & 15, b1 = (uint32_t)(uintptr_t)wb1 & 15;
+        const uint8_t *wa0 = wb0 - b0, *wa1 = wb1 - b1;
+        constexpr bool ALIGNED = MF::TS % 16 == 0;  // every row starts at the base's place in its 16 bytes
+        const uint32_t seg_all = MF::SBK == 32 ? (uint32_t)(MF::TS * KST) : (uint32_t)MF::TS;
         uint32_t wp_off[NTW], wp_p[NTW];
-        if constexpr (S::FAST) {
 #pragma unroll
-            for (int t = 0; t < NTW; t++) {
-                const int i0 = tid + S::NT * t, i = i0 < NP ? i0 : i0 - NP;
-                const int r = i / W::PCS;
-                wp_p[t] = (uint32_t)(i - r * W::PCS);
-                wp_off[t] = row_off(r, __builtin_amdgcn_readfirstlane(r / S::RPB));
-            }
+        for (int t = 0; t < NTW; t++) {
+            const int w0 = S::NT * t + 64 * wave, i = (w0 < NP ? w0 : w0 - NP) + lane;
+            const int r = i / W::PCS, m = S::NM > 1 ? __builtin_amdgcn_readfirstlane(r / S::RPB) : 0;
+            wp_p[t] = (uint32_t)(i - r * W::PCS);
+            wp_off[t] = row_off(r, m) + (m == 0 ? b0 : b1);
+            if constexpr (ALIGNED) wp_off[t] = (wp_off[t] & ~15u) + 16 * min(wp_p[t], ((m == 0 ? b0 : b1) + seg_all - 1) >> 4);
         }
-        auto issue_w = [&](int st_w, uint8_t *wbuf, int tido) __attribute__((always_inline)) {
-            const int nk_w = min(KST, n_ks - st_w * KST);
-            const uint32_t seg_w = MF::SBK == 32 ? MF::TS * nk_w : MF::TS;  // bytes of a row in this stage
+        auto issue_w = [&](int st_w, uint32_t wbuf) __attribute__((always_inline)) {
+            const uint32_t seg_w = MF::SBK == 32 ? MF::TS * min(KST, n_ks - st_w * KST) : MF::TS;  // bytes of a row in this stage
+            const uint32_t at = (uint32_t)(W::SEG * st_w);
 #pragma unroll
             for (int t = 0; t < NTW; t++) {
-                const int i0 = tido + S::NT * t, i = i0 < NP ? i0 : i0 - NP;  // the wrap is uniform across the wave
-                int m;
-                uint32_t o, p;
-                if constexpr (S::FAST) {
-                    m = S::NM > 1 ? __builtin_amdgcn_readfirstlane(i / (S::RPB * W::PCS)) : 0;
-                    o = wp_off[t];
-                    p = wp_p[t];
-                } else {
-                    const int r = i / W::PCS;
-                    p = (uint32_t)(i - r * W::PCS);
-                    m = __builtin_amdgcn_readfirstlane(r / S::RPB);
-                    o = row_off(r, m);
-                }
-                const uint8_t *mb = m == 0 ? wb0 : wb1;
-                o += (uint32_t)(W::SEG * st_w);                                // the row's stage bytes
-                const uint32_t mis = ((uint32_t)(uintptr_t)mb + o) & 15;      // ... from a 16-byte boundary
-                const uint32_t pc = min(p, (mis + seg_w - 1) >> 4);
-                // from the 16-byte boundary at or below the row's stage bytes, taken on the full
-                // address (a slot whose base is not 16-byte aligned has mis > o for its row 0)
-                const uint8_t *al = (const uint8_t *)(((uintptr_t)mb + o) & ~(uintptr_t)15);
-                dma16<S::ADMA>(al + 16 * pc, wbuf + (i - (tido & 63)) * 16);
+                const int w0 = S::NT * t + 64 * wave, wi = w0 < NP ? w0 : w0 - NP;  // the wave's first piece
+                const uint8_t *base = S::NM > 1 && wi >= S::RPB * W::PCS ? wa1 : wa0;
+                uint32_t o = wp_off[t] + at;
+                if constexpr (!ALIGNED) o = (o & ~15u) + 16 * min(wp_p[t], ((o & 15) + seg_w - 1) >> 4);
+                dma16_s(base, o, wbuf + 16 * wi);
             }
         };
-        // Activations of half-stage h (K-steps h*KA .. h*KA+KA-1, clamped to the row: a clamped load
-        // fills a slot nothing reads) into buffer h & 1, by the waves that own a pick block.
-        auto issue_a = [&](int h) __attribute__((always_inline)) {
-            if (stager) {
+        // K-steps KA*p .. KA*p + KA-1 of the row (clamped to it where it may end in between: unused) into a
+        // ring slot (an LDS address) of MBS pick blocks
+        auto issue_a = [&](int p, uint32_t slot, auto mbs_c) __attribute__((always_inline)) {
+            constexpr int MBS = decltype(mbs_c)::value;
+            if (!stager) return;
 #pragma unroll
-                for (int kk = 0; kk < S::KA; kk++)
-                    dma16<S::ADMA>(asrc + min(h * S::KA + kk, n_ks - 1) * 32, As + (h & 1) * S::A_HALF + ((kk * MF_MB + wave) * 64) * 16);
+            for (int kk = 0; kk < S::KA; kk++) {
+                const int ks = p * S::KA + kk;
+                dma16(asrc + (MF::SBK == 32 ? min(ks, n_ks - 1) : ks) * 32, slot + (kk * MBS + wave) * 1024);
             }
         };
-        // vmcnt(NTW) alone: every load but this wave's last NTW (the next stage's windows) is done
-        constexpr int WAIT_BUT_W = (NTW & 15) | ((NTW >> 4) << 14) | (7 << 4) | (15 << 8);
 
-        // Pipeline: the activations of the next half-stage load while this one computes (two
-        // buffers), and where two window buffers fit, the next stage's windows load during the whole
-        // stage. One barrier per half-stage both publishes its loads and frees the buffer they
-        // replace; a single window buffer needs a second barrier before it is refilled.
+        // this lane's rows: their start in global memory mod 16
+        uint32_t lmis[NB];
+#pragma unroll
+        for (int q = 0; q < NB; q++) lmis[q] = (mw == 0 ? b0 : b1) + (ALIGNED ? 0 : row_off(mw * S::RPB + wrow + 16 * q + l16, mw));
+
+        const uint32_t as_lds = lds_addr(As), ws_lds = lds_addr(Ws);
         const int st_lo = a.split_st ? blockIdx.y * a.split_st : 0;
         const int st_hi = a.split_st ? min(n_st, st_lo + a.split_st) : n_st;
-        issue_a(st_lo * S::HPS);
-        if constexpr (S::WDB) issue_w(st_lo, Ws + (st_lo & 1) * S::W_BYTES, tid);
-        for (int st = st_lo; st < st_hi; st++) {
-            // Per-lane addressing is recomputed from an opaque copy of the thread index each stage
-            // (a few integer operations) rather than kept in registers across the stage loop.
-            int tido = tid;
-            asm("" : "+v"(tido));
-            const int l16o = tido & 15;
-            const int nk = min(KST, n_ks - st * KST);              // K-steps in this stage
-            uint8_t *const Wst = Ws + (S::WDB ? (st & 1) * S::W_BYTES : 0);
-            if (st == st_lo && tid < MF_MT) {
-                meta_sa[tid] = my_sa;
-                meta_pick[tid] = my_pick;
+        // The stages, with the tile's count of 16-pick MFMA blocks as a constant. Pipeline: part p's
+        // activations are requested at part p - (NA - 1), stage st's windows at the start of stage
+        // st - (NWB - 1): a few hundred cycles of K-steps cover neither a round trip to L2 (the
+        // activations) nor one to HBM. One barrier per part publishes its loads and frees the ring slots
+        // that the loads issued after it overwrite. Near an item's end, where fewer loads are in flight
+        // than in_flight counts on, a part waits for all of them.
+        auto stages = [&](auto mbs_c) __attribute__((always_inline)) {
+            constexpr int MBS = decltype(mbs_c)::value, NA = S::na(MBS), SLOT = S::KA * MBS * 1024;
+            const int p_lo = st_lo * S::HPS, p_hi = st_hi * S::HPS;
+            // the loads before the first part, in the order that the parts before it would have issued them
+#pragma unroll
+            for (int q = 1 - NA < -(S::NWB - 1) * S::HPS ? 1 - NA : -(S::NWB - 1) * S::HPS; q < 0; q++) {
+                if (q + NA - 1 >= 0 && p_lo + q + NA - 1 < p_hi) issue_a(p_lo + q + NA - 1, as_lds + (q + NA - 1) * SLOT, mbs_c);
+                if (q % S::HPS == 0 && st_lo + q / S::HPS + S::NWB - 1 < st_hi)
+                    issue_w(st_lo + q / S::HPS + S::NWB - 1, ws_lds + (q / S::HPS + S::NWB - 1) * S::W_BYTES);
             }
-            if constexpr (!S::WDB) {
-                if (st != st_lo) __syncthreads();  // every wave is done with the previous stage's windows
-                issue_w(st, Wst, tido);
-            }
-            __builtin_amdgcn_s_waitcnt(0);  // this stage's windows and first activations
-            __syncthreads();
-            if (S::HPS >= 2)
-                issue_a(S::HPS * st + 1);
-            else if (st + 1 < st_hi)
-                issue_a(st + 1);
-            if constexpr (S::WDB)
-                if (st + 1 < st_hi) issue_w(st + 1, Ws + ((st + 1) & 1) * S::W_BYTES, tido);
+            int aslot = 0, wslot = 0;  // ring slots of the current part and stage
+            for (int st = st_lo; st < st_hi; st++) {
+                const int nk = min(KST, n_ks - st * KST);              // K-steps in this stage
+                const int nke = MF::SBK == 32 ? nk : KST;              // super-block formats: every stage is whole
+                uint8_t *const Wst = Ws + wslot * S::W_BYTES;
+                // the start of part hp: its loads are in, the next ones go out
+                const uint8_t *Ap;
+                auto start_part = [&](auto hp_c) __attribute__((always_inline)) {
+                    constexpr int hp = decltype(hp_c)::value;
+                    const int p = st * S::HPS + hp;
+                    const int last_w = (hp == 0 ? st - 1 : st) + S::NWB - 1;  // the last windows requested before this part
+                    if (p + NA - 2 < p_hi && last_w < st_hi) {
+                        constexpr int na = S::in_flight(hp, NA, NTW, S::KA), nb = S::in_flight(hp, NA, NTW, 0);
+                        if (stager) __builtin_amdgcn_s_waitcnt((na & 15) | ((na >> 4) << 14) | (7 << 4) | (15 << 8));
+                        else __builtin_amdgcn_s_waitcnt((nb & 15) | ((nb >> 4) << 14) | (7 << 4) | (15 << 8));
+                    } else {
+                        __builtin_amdgcn_s_waitcnt(0);
+                    }
+                    __syncthreads();
+                    const int prev = aslot == 0 ? NA - 1 : aslot - 1;  // freed by the barrier
+                    if (p + NA - 1 < p_hi) issue_a(p + NA - 1, as_lds + prev * SLOT, mbs_c);
+                    if (hp == 0 && st + S::NWB - 1 < st_hi) issue_w(st + S::NWB - 1, ws_lds + (wslot == 0 ? S::NWB - 1 : wslot - 1) * S::W_BYTES);
+                    Ap = As + aslot * SLOT;
+                    aslot = aslot + 1 == NA ? 0 : aslot + 1;
+                };
+                start_part(Ic<0>{});
 
-            // this lane's windows
-            const uint8_t *win[NM][NB];
-            WinRef wr[NM][NB];
-            typename MF::Stage stg[NM][NB];
+                // this lane's windows
+                const uint8_t *win[NM][NB];
+                WinRef wr[NM][NB];
+                typename MF::Stage stg[NM][NB];
 #pragma unroll
-            for (int m = 0; m < NM; m++)
+                for (int m = 0; m < NM; m++)
 #pragma unroll
-                for (int q = 0; q < NB; q++) {
-                    // this lane's row within the block's windows, and its start in global memory mod 16
-                    const int lrow = mw * S::RPB + wrow + 16 * q + l16o;
-                    const uint32_t lmis = (uint32_t)(uintptr_t)(mw == 0 ? wb0 : wb1) + row_off(lrow, mw);
-                    win[m][q] = Wst + lrow * W::BYTES + ((lmis + (uint32_t)(W::SEG * st)) & 15);
-                    wr[m][q] = WinRef::at<MF::ORG>(win[m][q]);
-                    stg[m][q].load(wr[m][q], grp);
+                    for (int q = 0; q < NB; q++) {
+                        win[m][q] = Wst + (mw * S::RPB + wrow + 16 * q + l16) * W::BYTES + ((lmis[q] + (uint32_t)(W::SEG * st)) & 15);
+                        wr[m][q] = WinRef::at<MF::ORG>(win[m][q]);
+                        stg[m][q].load(wr[m][q], grp);
+                    }
+
+                bool zero[NM][NB];
+                if constexpr (STEP) {
+#pragma unroll
+                    for (int m = 0; m < NM; m++)
+#pragma unroll
+                        for (int q = 0; q < NB; q++) zero[m][q] = false;
+                } else if constexpr (POW2) {
+#pragma unroll
+                    for (int m = 0; m < NM; m++)
+#pragma unroll
+                        for (int q = 0; q < NB; q++) {
+                            zero[m][q] = false;
+                            // the base is the largest block exponent of the item's stages so far: the
+                            // accumulators only ever move down onto a larger base (moving them up onto a
+                            // smaller one overflowed f32 for rows whose block scales span more than 2^127)
+                            int base = st > st_lo ? rb[m][q] : 0;
+#pragma unroll
+                            for (int kk = 0; kk < KST; kk++)
+                                if (kk < nk) base = max(base, (int)MF::expo(win[m][q], kk));
+                            if (st > st_lo && base != rb[m][q]) {
+#pragma unroll
+                                for (int mb = 0; mb < MBS; mb++)
+#pragma unroll
+                                    for (int i = 0; i < 4; i++) acc[m][q][mb][i] = ldexpf(acc[m][q][mb][i], rb[m][q] - base);
+                            }
+                            rb[m][q] = base;
+                        }
+                } else {
+#pragma unroll
+                    for (int m = 0; m < NM; m++)
+#pragma unroll
+                        for (int q = 0; q < NB; q++) {
+                            // the accumulators move onto the new scale at the start of the K-steps (only
+                            // the tile's pick blocks); a zero scale keeps the old one (its codes do not count)
+                            const float d = stg[m][q].d;
+                            zero[m][q] = d == 0.f;
+                            const float ratio = d != 0.f ? rs[m][q] * __builtin_amdgcn_rcpf(d) : 1.f;
+                            rs[m][q] = d != 0.f ? d : rs[m][q];
+#pragma unroll
+                            for (int mb = 0; mb < MBS; mb++) acc[m][q][mb] *= ratio;
+                        }
                 }
 
-            bool zero[NM][NB];
-            float ratio[NM][NB];  // running-scale moves of this stage (scale per super-block)
-            if constexpr (STEP) {
-#pragma unroll
-                for (int m = 0; m < NM; m++)
-#pragma unroll
-                    for (int q = 0; q < NB; q++) zero[m][q] = false;
-            } else if constexpr (POW2) {
-#pragma unroll
-                for (int m = 0; m < NM; m++)
-#pragma unroll
-                    for (int q = 0; q < NB; q++) {
-                        zero[m][q] = false;
-                        // the base is the largest block exponent of the item's stages so far: the
-                        // accumulators only ever move down onto a larger base (moving them up onto a
-                        // smaller one overflowed f32 for rows whose block scales span more than 2^127)
-                        int base = st > st_lo ? rb[m][q] : 0;
-#pragma unroll
-                        for (int kk = 0; kk < KST; kk++)
-                            if (kk < nk) base = max(base, (int)MF::expo(win[m][q], kk));
-                        if (st > st_lo && base != rb[m][q]) {
-#pragma unroll
-                            for (int mb = 0; mb < MF_MB; mb++)
-#pragma unroll
-                                for (int i = 0; i < 4; i++) acc[m][q][mb][i] = ldexpf(acc[m][q][mb][i], rb[m][q] - base);
-                        }
-                        rb[m][q] = base;
-                    }
-            } else {
-#pragma unroll
-                for (int m = 0; m < NM; m++)
-#pragma unroll
-                    for (int q = 0; q < NB; q++) {
-                        // the accumulators move onto the new scale at the start of the K-steps (only
-                        // the tile's pick blocks); a zero scale keeps the old one (its codes do not count)
-                        const float d = stg[m][q].d;
-                        zero[m][q] = d == 0.f;
-                        ratio[m][q] = d != 0.f ? rs[m][q] * __builtin_amdgcn_rcpf(d) : 1.f;
-                        rs[m][q] = d != 0.f ? d : rs[m][q];
-                    }
-            }
-
-            // The K-steps, with the tile's count of 16-pick MFMA blocks as a constant, software
-            // pipelined so that no step waits on an LDS read it issued itself: the window bytes of a
-            // step are requested two steps ahead, its table lookups and activation fragments one step
-            // ahead (step kk issues those of kk+1 once its own fragment is decoded, and they arrive
-            // while its MFMAs run). The first step of the second half-stage reads its activations
-            // after the barrier that publishes them. A scheduling fence closes each step (without
-            // it the compiler interleaves all eight steps and runs out of registers).
-            auto ksteps = [&](auto mbs_c) __attribute__((always_inline)) {
-                constexpr int MBS = decltype(mbs_c)::value;
-                const int nke = MF::SBK == 32 ? nk : KST;  // super-block formats: every stage is whole
+                // The K-steps, software pipelined so that no step waits on an LDS read it issued itself:
+                // the window bytes of a step are requested two steps ahead, its table lookups and
+                // activation fragments one step ahead (step kk issues those of kk+1 once its own fragment
+                // is decoded, and they arrive while its MFMAs run). The first step of a part reads its
+                // activations after the barrier that publishes them. A scheduling fence closes each step
+                // (without it the compiler interleaves all eight steps and runs out of registers).
                 typename MF::Raw rw[2][NM][NB];
                 typename MF::Look lk[2][NM][NB];
                 f16x8 av[2][MBS];
@@ -345,41 +367,20 @@ __global__ __launch_bounds__(1024, 4) void k_gmm(const MfArgs a) {
                         for (int q = 0; q < NB; q++) lk[kk & 1][m][q] = MF::look(rw[kk & 1][m][q], stg[m][q], kk, grp, tab, zero[m][q]);
                 };
                 auto issue_av = [&](int kk) __attribute__((always_inline)) {
-                    const uint8_t *Ak = As + ((S::HPS >= 2 ? kk / S::KA : st) & 1) * S::A_HALF + (kk % S::KA) * MF_MB * 64 * 16;
 #pragma unroll
-                    for (int mb = 0; mb < MBS; mb++) av[kk & 1][mb] = *(const f16x8 *)(Ak + (mb * 64 + lane) * 16);
+                    for (int mb = 0; mb < MBS; mb++) av[kk & 1][mb] = *(const f16x8 *)(Ap + (((kk % S::KA) * MBS + mb) * 64 + lane) * 16);
                 };
-                if constexpr (!STEP && !POW2) {
-#pragma unroll
-                    for (int m = 0; m < NM; m++)
-#pragma unroll
-                        for (int q = 0; q < NB; q++) {
-#pragma unroll
-                            for (int mb = 0; mb < MBS; mb++) acc[m][q][mb] *= ratio[m][q];
-                        }
-                }
                 issue_raw(0);
                 if (1 < nke) issue_raw(1);
                 if constexpr (S::PF) {
                     issue_look(0);
                     issue_av(0);
                 }
-#pragma unroll
-                for (int kk = 0; kk < KST; kk++) {
-                    if (kk >= nke) break;
-                    if (S::HPS >= 2 && kk > 0 && kk % S::KA == 0) {
-                        // a later part of the stage: its activations (loaded during the previous
-                        // part) are in. Only the first part's wait can leave the next stage's
-                        // windows in flight: later parts' activations were requested after them.
-                        if (S::WDB && st + 1 < st_hi && kk == S::KA)
-                            __builtin_amdgcn_s_waitcnt(WAIT_BUT_W);
-                        else
-                            __builtin_amdgcn_s_waitcnt(0);
-                        __syncthreads();
-                        if (kk / S::KA + 1 < S::HPS)
-                            issue_a(S::HPS * st + kk / S::KA + 1);
-                        else if (st + 1 < st_hi)
-                            issue_a(S::HPS * (st + 1));
+                auto step = [&](auto kk_c) __attribute__((always_inline)) {
+                    constexpr int kk = decltype(kk_c)::value;
+                    if (kk >= nke) return;  // uniform
+                    if constexpr (kk > 0 && kk % S::KA == 0) {
+                        start_part(Ic<kk / S::KA>{});
                         if constexpr (S::PF) issue_av(kk);
                     }
                     if constexpr (!S::PF) {
@@ -415,7 +416,7 @@ __global__ __launch_bounds__(1024, 4) void k_gmm(const MfArgs a) {
                     if (kk + 2 < KST && kk + 2 < nke) issue_raw(kk + 2);  // into the buffer step kk has just used
                     if (S::PF && kk + 1 < KST && kk + 1 < nke) {
                         issue_look(kk + 1);
-                        if (!(S::HPS >= 2 && (kk + 1) % S::KA == 0)) issue_av(kk + 1);
+                        if ((kk + 1) % S::KA != 0) issue_av(kk + 1);
                     }
 #pragma unroll
                     for (int mb = 0; mb < MBS; mb++)
@@ -426,71 +427,77 @@ __global__ __launch_bounds__(1024, 4) void k_gmm(const MfArgs a) {
                                 acc[m][q][mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[kk & 1][mb], bf[m][q], acc[m][q][mb], 0, 0, 0);
                             }
                     __builtin_amdgcn_sched_barrier(0);
+                };
+                step(Ic<0>{}); step(Ic<1>{}); step(Ic<2>{}); step(Ic<3>{});
+                if constexpr (KST > 4) { step(Ic<4>{}); step(Ic<5>{}); step(Ic<6>{}); step(Ic<7>{}); }
+                // a row's last stage may end before its later parts: their barriers all the same (they
+                // were requested, and their slots count)
+                if constexpr (MF::SBK == 32) {
+                    if constexpr (S::HPS > 1) if (nke <= S::KA) start_part(Ic<1>{});
+                    if constexpr (S::HPS > 2) if (nke <= 2 * S::KA) start_part(Ic<2>{});
+                    if constexpr (S::HPS > 3) if (nke <= 3 * S::KA) start_part(Ic<3>{});
                 }
-            };
-            switch (mbs) {
-            case 1: ksteps(Ic<1>{}); break;
-            case 2: ksteps(Ic<2>{}); break;
-            case 3: ksteps(Ic<3>{}); break;
-            case 4: ksteps(Ic<4>{}); break;
-            default: ksteps(Ic<5>{}); break;
+                wslot = wslot + 1 == S::NWB ? 0 : wslot + 1;
             }
+        };
+        switch (mbs) {
+        case 1: stages(Ic<1>{}); break;
+        case 2: stages(Ic<2>{}); break;
+        case 3: stages(Ic<3>{}); break;
+        case 4: stages(Ic<4>{}); break;
+        default: stages(Ic<5>{}); break;
         }
 
         // epilogue: lane holds picks 16*mb + 4*grp + i (i < 4) of weight row n (block q)
         float fs[NB];
 #pragma unroll
         for (int q = 0; q < NB; q++) fs[q] = POW2 ? ldexpf(1.0f, rb[0][q] - 128) : rs[0][q];
-        auto value = [&](int q, int mb, int i, float sa) __attribute__((always_inline)) {
-            return acc[0][q][mb][i] * fs[q] * sa;
-        };
         if constexpr (MODE == 0) {
-            // the up waves hand their values to the gate waves through LDS (the activation
-            // buffers, free once every wave is past the last K-step)
-            float *xu = (float *)As;
+            // The gate wave and the up wave of the same rows hand each other half of their values through
+            // LDS (the activation buffers, free once every wave is past the last K-step): the gate wave
+            // finishes rows 4*grp and 4*grp + 1 of each pick block, the up wave the other two.
+            float *xv = (float *)As;
             __syncthreads();
-            if (mw == 1) {
 #pragma unroll
-                for (int mb = 0; mb < MF_MB; mb++) {
-                    if (mb >= mbs) break;
+            for (int mb = 0; mb < MF_MB; mb++) {
+                if (mb >= mbs) break;
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const int r = 16 * mb + 4 * grp + i;
+                for (int i = 0; i < 2; i++) {
+                    const int r = 16 * mb + 4 * grp + (mw == 0 ? 2 : 0) + i;
 #pragma unroll
-                        for (int q = 0; q < NB; q++) xu[r * S::RPB + wrow + 16 * q + l16] = value(q, mb, i, meta_sa[r]);
-                    }
+                    for (int q = 0; q < NB; q++) xv[r * S::RPB + wrow + 16 * q + l16] = (mw == 0 ? acc[0][q][mb][2 + i] : acc[0][q][mb][i]) * fs[q] * meta_sa[r];
                 }
             }
             __syncthreads();
-            if (mw == 0) {
 #pragma unroll
-                for (int mb = 0; mb < MF_MB; mb++) {
-                    if (mb >= mbs) break;
+            for (int mb = 0; mb < MF_MB; mb++) {
+                if (mb >= mbs) break;
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const int r = 16 * mb + 4 * grp + i;
-                        if (r >= tile.m) continue;
-                        const int pos = tile.pos0 + r;
+                for (int i = 0; i < 2; i++) {
+                    const int r = 16 * mb + 4 * grp + (mw == 0 ? 0 : 2) + i;
+                    if (r >= tile.m) continue;
+                    const int pos = tile.pos0 + r;
 #pragma unroll
-                        for (int q = 0; q < NB; q++) {
-                            const int n = nblk * S::RPB + wrow + 16 * q + l16;
-                            if (n >= a.n) continue;
-                            // sigmoid(z) = 1 / (1 + 2^(-z log2 e)) on the hardware's exp2 and
-                            // reciprocal (each within 1 ulp)
-                            constexpr float LOG2E = 1.4426950408889634f;
-                            float g = value(q, mb, i, meta_sa[r]), u = xu[r * S::RPB + wrow + 16 * q + l16], o;
-                            if (a.act == CW_ACT_SILU) {
-                                o = g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-g * LOG2E)) * u;
-                            } else {
-                                const int64_t e = tile.expert;  // every pick of the tile's
-                                if (a.bias0) g += a.bias0[e * a.n + n];
-                                if (a.bias1) u += a.bias1[e * a.n + n];
-                                g = fminf(g, a.limit);
-                                u = fminf(fmaxf(u, -a.limit), a.limit);
-                                o = (u + 1.0f) * (g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-(g * a.alpha) * LOG2E)));
-                            }
-                            a.h[(int64_t)pos * a.ldh + n] = o;
+                    for (int q = 0; q < NB; q++) {
+                        const int n = nblk * S::RPB + wrow + 16 * q + l16;
+                        if (n >= a.n) continue;
+                        const float own = (mw == 0 ? acc[0][q][mb][i] : acc[0][q][mb][2 + i]) * fs[q] * meta_sa[r];
+                        const float other = xv[r * S::RPB + wrow + 16 * q + l16];
+                        // sigmoid(z) = 1 / (1 + 2^(-z log2 e)) on the hardware's exp2 and
+                        // reciprocal (each within 1 ulp)
+                        constexpr float LOG2E = 1.4426950408889634f;
+                        float g = mw == 0 ? own : other, u = mw == 0 ? other : own, o;
+                        if (a.act == CW_ACT_SILU) {
+                            o = g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-g * LOG2E)) * u;
+                        } else {
+                            const int64_t e = tile.expert;  // every pick of the tile's
+                            if (a.bias0) g += a.bias0[e * a.n + n];
+                            if (a.bias1) u += a.bias1[e * a.n + n];
+                            g = fminf(g, a.limit);
+                            u = fminf(fmaxf(u, -a.limit), a.limit);
+                            o = (u + 1.0f) * (g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-(g * a.alpha) * LOG2E)));
                         }
+                        a.h[(int64_t)pos * a.ldh + n] = o;
                     }
                 }
             }
@@ -509,7 +516,7 @@ __global__ __launch_bounds__(1024, 4) void k_gmm(const MfArgs a) {
                         const int n = nblk * S::RPB + wrow + 16 * q + l16;
                         if (n >= a.n) continue;
                         float *p = a.dn + blockIdx.y * a.split_stride + (int64_t)pick * a.n + n;
-                        const float v = value(q, mb, i, meta_sa[r]);
+                        const float v = acc[0][q][mb][i] * fs[q] * meta_sa[r];
                         if (split)
                             __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // at the coherence point
                         else
@@ -827,7 +834,7 @@ template <class MF, int MODE>
 static int launch(const MfArgs &a, int tiles_max, int splits, hipStream_t s) {
     using S = GmShape<MF, MODE>;
     if (a.k % MF::SBK) return set_error(CW_ENOTSUP, "mfma: k %d is not a multiple of %d", a.k, MF::SBK);
-    if ((int64_t)a.n * a.row_bytes >= ((int64_t)1 << 32))
+    if ((int64_t)a.n * a.row_bytes > ((int64_t)1 << 32) - 16)  // (32-bit offsets from the 16-byte boundary below the matrix)
         return set_error(CW_ENOTSUP, "mfma: a matrix of %d rows of %lld bytes is 4 GiB or more", a.n, (long long)a.row_bytes);
     const int R = run_of_tiles(tiles_max);
     const int64_t items = gemm_items(tiles_max, S::RPB, a.n);
@@ -960,8 +967,8 @@ __global__ __launch_bounds__(64 * W) void k_skinny_q4k(const uint8_t *w, int64_t
 #pragma unroll
     for (int t = 0; t < NI; t++) {
         const int c = min(64 * t + lane, NCH - 1), r = c / (RB / 16), piece = c - r * (RB / 16), j = piece / 9;
-        dma16<true>(w + (int64_t)min(blockIdx.x * 16 + r, n - 1) * row_bytes + 144 * min(s0 + j, nsb - 1) + 16 * (piece - 9 * j),
-                    &wl[wave][1024 * t]);
+        dma16(w + (int64_t)min(blockIdx.x * 16 + r, n - 1) * row_bytes + 144 * min(s0 + j, nsb - 1) + 16 * (piece - 9 * j),
+              lds_addr(&wl[wave][1024 * t]));
     }
     uint4 head[SKINNY_SB];
     uint2 qs[SKINNY_SB][4];

@@ -222,6 +222,7 @@ __global__ __launch_bounds__(512, 4) void k_gms(const MfArgs a) {
             const int n = nblk * S::RPB + (r - m * S::RPB);
             return (uint32_t)(n < a.n ? n : 0) * (uint32_t)a.row_bytes;
         };
+        const uint32_t as_lds = lds_addr(As), ws_lds = lds_addr(Ws);
         auto issue_w = [&](int st) __attribute__((always_inline)) {
             const uint32_t seg = SF::SBK == 32 ? SF::TS * min(KST, n_ks - st * KST) : SF::TS;
             constexpr int NP = S::NM * S::RPB * S::PCS;
@@ -238,22 +239,22 @@ __global__ __launch_bounds__(512, 4) void k_gms(const MfArgs a) {
                 const int m = S::NM > 1 ? __builtin_amdgcn_readfirstlane(r / S::RPB) : 0;
                 const uint8_t *at = (m == 0 ? wb0 : wb1) + row_off(r, m) + (uint32_t)(S::SEG * st);
                 const uint32_t mis = (uint32_t)(uintptr_t)at & 15, pc = min((uint32_t)p, (mis + seg - 1) >> 4);
-                dma16<true>(at - mis + 16 * pc, Ws + (i - (tido & 63)) * 16);
+                dma16(at - mis + 16 * pc, ws_lds + 16 * (S::NT * t + 64 * wave));
             }
         };
         // part p of stage st: K-steps KA p .. (clamped to the row: unused), hi and lo; or the sums
         auto issue_a = [&](int st, int p, int buf) __attribute__((always_inline)) {
             if (!stager) return;
-            uint8_t *dst = As + buf * S::PART + wave * 1024;
+            const uint32_t dst = as_lds + buf * S::PART + wave * 1024;
             if (SF::MIN && p == KST / KA) {
-                dma16<true>(asrc + 2 * a.k + 32 * st, dst);
+                dma16(asrc + 2 * a.k + 32 * st, dst);
                 return;
             }
 #pragma unroll
             for (int kk = 0; kk < KA; kk++) {
                 const int ks = min(st * KST + p * KA + kk, n_ks - 1);
-                dma16<true>(asrc + 32 * ks, dst + (2 * kk) * MF_MB * 1024);
-                dma16<true>(asrc + a.k + 32 * ks, dst + (2 * kk + 1) * MF_MB * 1024);
+                dma16(asrc + 32 * ks, dst + (2 * kk) * MF_MB * 1024);
+                dma16(asrc + a.k + 32 * ks, dst + (2 * kk + 1) * MF_MB * 1024);
             }
         };
 
