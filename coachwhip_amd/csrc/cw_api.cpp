@@ -102,7 +102,7 @@ static bool qmatmul_mfma(int dtype, int64_t k, int64_t m) {
 // call stays on the matvec. CWMOE_MM_MIN_ROWS (rows) overrides.
 static bool qmatmul_split(int dtype, int64_t n, int64_t k, int64_t m) {
     if ((dtype != CW_Q5_K && dtype != CW_Q6_K) || m >= (1 << 24) || k % 256 || k > 8192 || n <= 0 || n >= (1ll << 31) ||
-        n * (k / 256 * cw_type_size(dtype)) >= (1ll << 32))
+        n * (k / 256 * cw_type_size(dtype)) > (1ll << 32) - 16)
         return false;
     if (const char *e = getenv("CWMOE_MM_MIN_ROWS")) return m >= atoll(e);
     return m > 2 && (5 * m - 12) * n * k >= 215000000ll;

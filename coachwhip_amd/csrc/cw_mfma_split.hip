@@ -223,25 +223,35 @@ __global__ __launch_bounds__(512, 4) void k_gms(const MfArgs a) {
             return (uint32_t)(n < a.n ? n : 0) * (uint32_t)a.row_bytes;
         };
         const uint32_t as_lds = lds_addr(As), ws_lds = lds_addr(Ws);
-        auto issue_w = [&](int st) __attribute__((always_inline)) {
-            const uint32_t seg = SF::SBK == 32 ? SF::TS * min(KST, n_ks - st * KST) : SF::TS;
-            constexpr int NP = S::NM * S::RPB * S::PCS;
-            static_assert(NP % 64 == 0, "a wave's pieces are whole");
-            // an opaque thread index: the pieces' addresses are worked out per stage, not kept across it
-            int tido = tid;
-            asm("" : "+v"(tido));
-            // (uniform per wave: the last round's waves past the pieces leave)
+        // windows as in k_gmm: each piece's row and place once per tile, 32-bit offsets from the 16-byte
+        // boundary below the matrix
+        constexpr int NP = S::NM * S::RPB * S::PCS, NTW = (NP + S::NT - 1) / S::NT;
+        static_assert(S::RPB * S::PCS % 64 == 0, "a wave's pieces lie in one matrix");
+        const uint32_t b0 = (uint32_t)(uintptr_t)wb0 & 15, b1 = (uint32_t)(uintptr_t)wb1 & 15;
+        const uint8_t *wa0 = wb0 - b0, *wa1 = wb1 - b1;
+        constexpr bool ALIGNED = SF::TS % 16 == 0;
+        uint32_t wp_off[NTW], wp_p[NTW];
 #pragma unroll
-            for (int t = 0; t < (NP + S::NT - 1) / S::NT; t++) {
-                const int i = tido + S::NT * t;
-                if (S::NT * t + 64 * wave >= NP) break;
-                const int r = i / S::PCS, p = i - r * S::PCS;
-                const int m = S::NM > 1 ? __builtin_amdgcn_readfirstlane(r / S::RPB) : 0;
-                const uint8_t *at = (m == 0 ? wb0 : wb1) + row_off(r, m) + (uint32_t)(S::SEG * st);
-                const uint32_t mis = (uint32_t)(uintptr_t)at & 15, pc = min((uint32_t)p, (mis + seg - 1) >> 4);
-                dma16(at - mis + 16 * pc, ws_lds + 16 * (S::NT * t + 64 * wave));
+        for (int t = 0; t < NTW; t++) {
+            const int w0 = S::NT * t + 64 * wave, i = (w0 < NP ? w0 : w0 - NP) + lane;
+            const int r = i / S::PCS, m = S::NM > 1 ? __builtin_amdgcn_readfirstlane(r / S::RPB) : 0;
+            wp_p[t] = (uint32_t)(i - r * S::PCS);
+            wp_off[t] = row_off(r, m) + (m == 0 ? b0 : b1);
+            if constexpr (ALIGNED) wp_off[t] = (wp_off[t] & ~15u) + 16 * min(wp_p[t], ((m == 0 ? b0 : b1) + S::SEG - 1) >> 4);
+        }
+        auto issue_w = [&](int st) __attribute__((always_inline)) {
+            const uint32_t seg = SF::SBK == 32 ? SF::TS * min(KST, n_ks - st * KST) : SF::TS, at = (uint32_t)(S::SEG * st);
+#pragma unroll
+            for (int t = 0; t < NTW; t++) {
+                const int w0 = S::NT * t + 64 * wave;
+                if (w0 >= NP) break;  // uniform per wave: the last round's waves past the pieces
+                uint32_t o = wp_off[t] + at;
+                if constexpr (!ALIGNED) o = (o & ~15u) + 16 * min(wp_p[t], ((o & 15) + seg - 1) >> 4);
+                dma16_s(S::NM > 1 && w0 >= S::RPB * S::PCS ? wa1 : wa0, o, ws_lds + 16 * w0);
             }
         };
+        // this lane's row: its start in global memory mod 16
+        const uint32_t lmis = (mw == 0 ? b0 : b1) + (ALIGNED ? 0 : row_off(mw * S::RPB + wrow + l16, mw));
         // part p of stage st: K-steps KA p .. (clamped to the row: unused), hi and lo; or the sums
         auto issue_a = [&](int st, int p, int buf) __attribute__((always_inline)) {
             if (!stager) return;
@@ -252,7 +262,7 @@ __global__ __launch_bounds__(512, 4) void k_gms(const MfArgs a) {
             }
 #pragma unroll
             for (int kk = 0; kk < KA; kk++) {
-                const int ks = min(st * KST + p * KA + kk, n_ks - 1);
+                const int ks = SF::SBK == 32 ? min(st * KST + p * KA + kk, n_ks - 1) : st * KST + p * KA + kk;
                 dma16(asrc + 32 * ks, dst + (2 * kk) * MF_MB * 1024);
                 dma16(asrc + a.k + 32 * ks, dst + (2 * kk + 1) * MF_MB * 1024);
             }
@@ -269,9 +279,7 @@ __global__ __launch_bounds__(512, 4) void k_gms(const MfArgs a) {
                 if (st != st_lo) __syncthreads();  // every wave is done with the previous stage's windows
                 issue_w(st);
                 const int nk = min(KST, n_ks - st * KST);
-                const int lrow = mw * S::RPB + wrow + l16;
-                const uint32_t mis = ((uint32_t)(uintptr_t)(mw == 0 ? wb0 : wb1) + row_off(lrow, mw) + (uint32_t)(S::SEG * st)) & 15;
-                const WinRef w = WinRef::at<0>(Ws + lrow * S::WB + mis);
+                const WinRef w = WinRef::at<0>(Ws + (mw * S::RPB + wrow + l16) * S::WB + ((lmis + (uint32_t)(S::SEG * st)) & 15));
                 typename SF::Stage stg;
                 f32x4 acc[MBS];
 #pragma unroll
@@ -339,30 +347,29 @@ __global__ __launch_bounds__(512, 4) void k_gms(const MfArgs a) {
         // epilogue: lane holds picks 16 mb + 4 grp + i of weight row n
         const int n = nblk * S::RPB + wrow + l16;
         if constexpr (MODE == 0) {
-            // up's values to the gate waves through the activation buffers
-            float *xu = (float *)As;
+            // half of the values each way between the gate and the up wave of the same rows, as in k_gmm
+            float *xv = (float *)As;
             __syncthreads();
-            if (mw == 1) {
 #pragma unroll
-                for (int mb = 0; mb < MF_MB; mb++) {
-                    if (mb >= mbs) break;
+            for (int mb = 0; mb < MF_MB; mb++) {
+                if (mb >= mbs) break;
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const int r = 16 * mb + 4 * grp + i;
-                        xu[r * S::RPB + wrow + l16] = tot[mb][i] * meta_sa[r];
-                    }
+                for (int i = 0; i < 2; i++) {
+                    const int r = 16 * mb + 4 * grp + (mw == 0 ? 2 : 0) + i;
+                    xv[r * S::RPB + wrow + l16] = (mw == 0 ? tot[mb][2 + i] : tot[mb][i]) * meta_sa[r];
                 }
             }
             __syncthreads();
-            if (mw == 0 && n < a.n) {
+            if (n < a.n) {
 #pragma unroll
                 for (int mb = 0; mb < MF_MB; mb++) {
                     if (mb >= mbs) break;
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const int r = 16 * mb + 4 * grp + i;
+                    for (int i = 0; i < 2; i++) {
+                        const int r = 16 * mb + 4 * grp + (mw == 0 ? 0 : 2) + i;
                         if (r >= tile.m) continue;
-                        float g = tot[mb][i] * meta_sa[r], u = xu[r * S::RPB + wrow + l16], o;
+                        const float own = (mw == 0 ? tot[mb][i] : tot[mb][2 + i]) * meta_sa[r], other = xv[r * S::RPB + wrow + l16];
+                        float g = mw == 0 ? own : other, u = mw == 0 ? other : own, o;
                         if (a.act == CW_ACT_SILU) {
                             o = g / (1.0f + expf(-g)) * u;
                         } else {
@@ -492,7 +499,7 @@ template <class SF, int MODE>
 static int launch(const MfArgs &a, int tiles_max, int splits, hipStream_t s) {
     using S = SpShape<SF, MODE>;
     if (a.k % SF::SBK) return set_error(CW_ENOTSUP, "mfma: k %d is not a multiple of %d", a.k, SF::SBK);
-    if ((int64_t)a.n * a.row_bytes >= ((int64_t)1 << 32))
+    if ((int64_t)a.n * a.row_bytes > ((int64_t)1 << 32) - 16)  // (32-bit offsets from the 16-byte boundary below the matrix)
         return set_error(CW_ENOTSUP, "mfma: a matrix of %d rows of %lld bytes is 4 GiB or more", a.n, (long long)a.row_bytes);
     MfArgs b = a;
     int64_t items;

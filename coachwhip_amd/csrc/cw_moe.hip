@@ -149,7 +149,7 @@ static bool split_path(const cw_moe_desc *d, int T) {
     const int P = d->pad > d->inter ? d->pad : d->inter;
     const int64_t gu = (int64_t)d->inter * (d->hidden / cw_block_size(d->dtype[0])) * cw_type_size(d->dtype[0]);
     const int64_t dn = (int64_t)d->hidden * (P / cw_block_size(d->dtype[2])) * cw_type_size(d->dtype[2]);
-    if (gu >= ((int64_t)1 << 32) || dn >= ((int64_t)1 << 32) || (int64_t)T * d->top_k >= (1 << 28)) return false;
+    if (gu > ((int64_t)1 << 32) - 16 || dn > ((int64_t)1 << 32) - 16 || (int64_t)T * d->top_k >= (1 << 28)) return false;
     if (getenv("CWMOE_PREFILL_MIN_TOKENS")) return T >= prefill_min_tokens();
     const double K = d->top_k, E = std::max<double>(d->slot_table ? d->n_slots : d->n_experts, K), distinct = E * (1 - pow(1 - K / E, T));
     return (T * K - distinct) * d->hidden * (2.0 * d->inter + P) >= 230e6;
