@@ -136,7 +136,14 @@ __device__ __forceinline__ void gx_dma16(const uint8_t *base, uint32_t off, uint
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base),
                  "s"(__builtin_amdgcn_readfirstlane(lds_base)) : "memory", "m0");
 }
-// the same for 4 bytes (base 4-byte aligned; lane l writes lds_base + 4 l)
+// the same if on > 0 (on wave-uniform, in a scalar register): the branch stays inside the asm, so that
+// the code around it is one basic block and its order of loads, reads and MFMAs is kept
+__device__ __forceinline__ void gx_dma16_if(const uint8_t *base, uint32_t off, uint32_t lds_base, int on) {
+    asm volatile("s_cmp_lt_i32 %3, 1\n\ts_cbranch_scc1 .Lgx_dma_%=\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1\n"
+                 ".Lgx_dma_%=:" : : "v"(off), "s"(base), "s"(__builtin_amdgcn_readfirstlane(lds_base)),
+                 "s"(__builtin_amdgcn_readfirstlane(on)) : "memory", "m0", "scc");
+}
+// the same as gx_dma16 for 4 bytes (base 4-byte aligned; lane l writes lds_base + 4 l)
 __device__ __forceinline__ void gx_dma4(const uint8_t *base, uint32_t off, uint32_t lds_base) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" : : "v"(off), "s"(base),
                  "s"(__builtin_amdgcn_readfirstlane(lds_base)) : "memory", "m0");
@@ -172,10 +179,15 @@ __device__ __forceinline__ void gx_wait_vm(int n) {
 // groups from whole 1 KB loads of their own. The activation operands of a
 // stage (token block t: its 16 tokens' 304-byte step records, whole) go to LDS by direct loads
 // too, two stages ahead (two buffers), issued by the first waves. Each wave reads the operands of
-// the next stage from LDS while it computes the current one: a token block's activation operands
-// right after that block's MFMAs, the weight operands at the end of the stage, so that their
-// latency hides behind the matrix work. One barrier per stage publishes every wave's loads (each
-// wave first waits for exactly its own).
+// the next stage from LDS between the MFMAs of the current one: a term's activation operands right
+// after its MFMAs, the weight operands, whose dwords the shift into the A operands has freed,
+// fragment by fragment over the stage, so that their latency hides behind the matrix work. (With a
+// token block's reads behind all of its MFMAs and the weight reads at the stage's end, the LDS
+// waited for the matrix cores and these for the LDS: a layer of 2,048 tokens over 128 experts of
+// 2880 x 2880 658 us, now 602; its MFMAs alone are 160, its weights at the rate of a large copy 350.)
+// One barrier per stage publishes every wave's loads (each wave first waits for exactly its own).
+// What bounds it: two waves per SIMD issue in order, 31% of their cycles waiting for the matrix
+// pipe, 31% at the barrier and for the LDS, 38% issuing.
 template <int MODE, int L = 0>
 struct GxShape {
     static constexpr int NW = 8, NT = 64 * NW;
@@ -268,6 +280,7 @@ __device__ __forceinline__ void gx_item(const MfArgs &a, const MfTile &tile, int
     // pieces, piece p (token p / 19, its piece p % 19) brought by lane p % 64 of load p / 64 (the
     // last load's lanes past piece 303 bring that piece again, into the block's padding)
     const bool stager = wave < mbs;
+    const int n_stx = stager ? n_st : 0;  // the stages it stages
     uint32_t xo[5] = {0, 0, 0, 0, 0};
     if (stager) {
 #pragma unroll
@@ -285,87 +298,94 @@ __device__ __forceinline__ void gx_item(const MfArgs &a, const MfTile &tile, int
     const int nw = (S::W_INST - wave + 7) / 8;
     int issued = 0;                    // this wave's loads in the item (it starts drained)
     int m_w0 = 0, m_a0 = 0;            // the count after stage 0's window and activation loads
-    // window loads of stage st into buffer st % 3 (this wave's share)
-    auto issue_w = [&](int st) __attribute__((always_inline)) {
-        const int buf = st % S::WDEPTH;
-        const uint32_t Wd = lds0 + buf * S::W_BYTES;
+    // window load j of stage st into buffer st % 3 (this wave's share: j < NJW), if on > 0
+    auto issue_w1 = [&](int st, int j, int on) __attribute__((always_inline)) {
+        const int wi = wave + 8 * j;
+        const uint32_t Wd = lds0 + (uint32_t)(st % S::WDEPTH) * S::W_BYTES + wi * 1024;
         if constexpr (L == 1) {
-            const int cb = min(4, nblk - 4 * st);  // blocks per row in this stage
-#pragma unroll
-            for (int j = 0; j < S::NJW; j++) {
-                const int wi = wave + 8 * j;
-                if (wi < S::W_INST) {
-                    const bool m1 = S::NM > 1 && wi >= S::MI;
-                    gx_dma16(m1 ? wa1 : wa0, cb == 4 ? wo[j] + 1088u * (uint32_t)st : wp[j], Wd + wi * 1024);
-                    issued++;
-                }
-            }
-            if (st == 0) m_w0 = issued;
-            return;
+            const bool m1 = S::NM > 1 && wi >= S::MI;
+            // a full stage's blocks, or a last stage's
+            gx_dma16_if(m1 ? wa1 : wa0, nblk - 4 * st >= 4 ? wo[j] + 1088u * (uint32_t)st : wp[j], Wd, wi < S::W_INST ? on : 0);
+        } else {
+            const uint32_t seg = 17u * (uint32_t)min(4, nblk - 4 * st);  // bytes of a row in this stage
+            const bool m1 = S::NM > 1 && wi >= S::W_INST / 2;
+            // the row's bytes of stage st start at o past the aligned base
+            const uint32_t o = wo[j] + 68u * (uint32_t)st + (m1 ? wm1 : wm0);
+            const uint32_t pc = min(wp[j], ((o & 15u) + seg - 1) >> 4);
+            gx_dma16_if(m1 ? wa1 : wa0, (o & ~15u) + 16 * pc, Wd, wi < S::W_INST ? on : 0);
         }
-        const uint32_t seg = 17u * (uint32_t)min(4, nblk - 4 * st);  // bytes of a row in this stage
+    };
+    auto issue_w = [&](int st) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < S::NJW; j++) {
-            const int wi = wave + 8 * j;
-            if (wi < S::W_INST) {
-                const bool m1 = S::NM > 1 && wi >= S::W_INST / 2;
-                // the row's bytes of stage st start at o past the aligned base
-                const uint32_t o = wo[j] + 68u * (uint32_t)st + (m1 ? wm1 : wm0);
-                const uint32_t pc = min(wp[j], ((o & 15u) + seg - 1) >> 4);
-                gx_dma16(m1 ? wa1 : wa0, (o & ~15u) + 16 * pc, Wd + wi * 1024);
-                issued++;
-            }
-        }
+        for (int j = 0; j < S::NJW; j++) issue_w1(st, j, 1);
+        issued += nw;
         if (st == 0) m_w0 = issued;
     };
-    // a stager's token block of stage st into activation buffer st % 2 (five 1 KB direct loads)
+    // a stager's load c (of five, 1 KB each) of its token block of stage st into activation buffer st % 2
+    auto issue_x1 = [&](int st, int c, int on) __attribute__((always_inline)) {
+        gx_dma16_if(a.ap, xo[c] + 304u * (uint32_t)st, Al + (uint32_t)(st & 1) * S::A_BYTES + wave * S::TB_BYTES + 1024 * c, on);
+    };
     auto issue_x = [&](int st) __attribute__((always_inline)) {
-        if (stager) {
-            const uint32_t d = Al + (st & 1) * S::A_BYTES + wave * S::TB_BYTES;
 #pragma unroll
-            for (int c = 0; c < 5; c++) gx_dma16(a.ap, xo[c] + 304u * (uint32_t)st, d + 1024 * c);
-            issued += 5;
-        }
+        for (int c = 0; c < 5; c++) issue_x1(st, c, n_stx);
+        if (stager) issued += 5;
         if (st == 0) m_a0 = issued;
+    };
+    // the loads a wave sends out in stage st, in order: its activations of st + 2, then its windows of st + 3
+    constexpr int N_LOADS = 5 + S::NJW;
+    // three token blocks' MFMAs hide the loads issued between them (602 us for a layer of 2,048 tokens
+    // over 128 experts of 2880 x 2880, against 607 with all of them first); fewer do not (a layer of
+    // 100 tokens: 385 us spread, 353 first)
+    constexpr bool SPREAD = NTB > 2;
+    auto issue_next = [&](int st, int i) __attribute__((always_inline)) {
+        if (i < 5) issue_x1(st + 2, i, n_stx - (st + 2));
+        else issue_w1(st + 3, i - 5, n_st - (st + 3));
     };
 
     // operands in registers: each token block's activations of the stage being computed, the raw
-    // weight dwords (5 around the block, and its E8M0 byte) of the next stage
+    // weight dwords of the next stage (the five that hold a block's 17 bytes, its E8M0 byte first)
     i32x8 bo[NB][3];  // an FP6 operand is dwords 0..5; the instruction ignores 6 and 7
     int bsc[NB];
-    uint32_t ra[S::NF][5], re[S::NF];
-    auto read_b = [&](int t, int st) __attribute__((always_inline)) {
-        // this lane's token's record: per term 16 code bytes of its K-group at 96 j + 16 grp and 8
-        // at 96 j + 64 + 8 grp, its scale dword at 288 + 4 grp (bank-conflict free: records are 76
-        // dwords apart)
-        const uint8_t *r = Ab + (st & 1) * S::A_BYTES + (tb0 + t) * S::TB_BYTES + 304 * l16;
-#pragma unroll
-        for (int j = 0; j < 3; j++) {
-            const i32x4 l = *(const i32x4 *)(r + 96 * j + 16 * grp);
-            const i32x2 h = *(const i32x2 *)(r + 96 * j + 64 + 8 * grp);
-            bo[t][j] = __builtin_shufflevector(l, __builtin_shufflevector(h, h, 0, 1, -1, -1), 0, 1, 2, 3, 4, 5, -1, -1);
-        }
-        bsc[t] = *(const int *)(r + 288 + 4 * grp);
+    uint32_t ra[S::NF][5];
+    // this lane's token's record of stage st in the wave's first token block, at its K-group's 16
+    // code bytes: per term 16 bytes at 96 j + 16 grp and 8 at 96 j + 64 + 8 grp, and the scale
+    // dword at 288 + 4 grp (bank-conflict free: records are 76 dwords apart). An offset from the
+    // LDS base, opaque so that one register serves every read of the stage.
+    auto b_off = [&](int st) __attribute__((always_inline)) {
+        uint32_t o = (uint32_t)(S::WDEPTH * S::W_BYTES + (st & 1) * S::A_BYTES + tb0 * S::TB_BYTES) + 304u * l16 + 16u * grp;
+        asm volatile("" : "+v"(o));
+        return o;
     };
-    // LDS offset of the E8M0 byte of this lane's block of fragment f in stage st's window
-    auto aoff = [&](int f, int st) __attribute__((always_inline)) -> uint32_t {
+    auto read_b1 = [&](int t, int j, uint32_t o) __attribute__((always_inline)) {
+        const uint8_t *r = smem + o + t * S::TB_BYTES;
+        const i32x4 l = *(const i32x4 *)(r + 96 * j);
+        const i32x2 h = *(const i32x2 *)(r - 8u * grp + 96 * j + 64);
+        bo[t][j] = __builtin_shufflevector(l, __builtin_shufflevector(h, h, 0, 1, -1, -1), 0, 1, 2, 3, 4, 5, -1, -1);
+    };
+    auto read_bs = [&](int t, uint32_t o) __attribute__((always_inline)) {
+        bsc[t] = *(const int *)(smem + o - 12u * grp + t * S::TB_BYTES + 288);
+    };
+    // LDS offset of this lane's block of fragment f in stage st's window (its E8M0 byte). L = 1:
+    // fragments are whole groups of 16 rows (272 cb bytes) apart, so their blocks share one
+    // alignment
+    auto a_off = [&](int st) __attribute__((always_inline)) {
+        uint32_t o = 0;
         if constexpr (L == 1) {
-            const int lr = rg * S::RW + 16 * (f % S::FR) + l16, cb = min(4, nblk - 4 * st);
-            return (uint32_t)((f / S::FR) * S::MI * 1024) + (uint32_t)lr * (17u * (uint32_t)cb) + 17u * grp;
+            o = (uint32_t)(rg * S::RW + l16) * (17u * (uint32_t)min(4, nblk - 4 * st)) + 17u * grp;
+            asm volatile("" : "+v"(o));
         }
-        const int lrow = (f / S::FR) * S::RPB + rg * S::RW + 16 * (f % S::FR) + l16;
-        return (uint32_t)lrow * (S::PCS * 16) + ((lmis[f] + 4u * (uint32_t)st) & 15u) + 17u * grp;
+        return o;
     };
-    auto read_a = [&](int st) __attribute__((always_inline)) {
-        const uint8_t *Wd = Wb + (st % S::WDEPTH) * S::W_BYTES;
+    auto aoff = [&](int f, int st, uint32_t o) __attribute__((always_inline)) -> uint32_t {
+        const uint32_t m = (uint32_t)(f / S::FR), fr = (uint32_t)(f % S::FR);
+        if constexpr (L == 1) return o + m * (S::MI * 1024) + fr * (272u * (uint32_t)min(4, nblk - 4 * st));
+        const uint32_t lrow = m * S::RPB + (uint32_t)rg * S::RW + 16 * fr + l16;
+        return lrow * (S::PCS * 16) + ((lmis[f] + 4u * (uint32_t)st) & 15u) + 17u * grp;
+    };
+    auto read_a1 = [&](int f, int st, uint32_t o) __attribute__((always_inline)) {
+        const uint32_t *q = (const uint32_t *)(smem + (st % S::WDEPTH) * S::W_BYTES + (aoff(f, st, o) & ~3u));
 #pragma unroll
-        for (int f = 0; f < S::NF; f++) {
-            const uint32_t off = aoff(f, st), cb = off + 1;
-            const uint32_t *q = (const uint32_t *)(Wd + (cb & ~3u));
-#pragma unroll
-            for (int i = 0; i < 5; i++) ra[f][i] = q[i];
-            re[f] = Wd[off];
-        }
+        for (int i = 0; i < 5; i++) ra[f][i] = q[i];
     };
 
     f32x4v acc[S::NF][NB];
@@ -398,9 +418,15 @@ __device__ __forceinline__ void gx_item(const MfArgs &a, const MfTile &tile, int
     gx_wait_vm(issued - (m_w0 > m_a0 ? m_w0 : m_a0));  // this wave's loads of stage 0
     __syncthreads();                                    // everyone's
     if constexpr (NTB > 0) {
+        const uint32_t ob = b_off(0), oa = a_off(0);
 #pragma unroll
-        for (int t = 0; t < NTB; t++) read_b(t, 0);
-        read_a(0);
+        for (int t = 0; t < NTB; t++) {
+#pragma unroll
+            for (int j = 0; j < 3; j++) read_b1(t, j, ob);
+            read_bs(t, ob);
+        }
+#pragma unroll
+        for (int f = 0; f < S::NF; f++) read_a1(f, 0, oa);
     }
     // Per stage st (its operands in registers): the activation loads of st + 2 and the window loads
     // of st + 3 go out, and the MFMAs of st run with the reads of st + 1's operands between them.
@@ -412,28 +438,33 @@ __device__ __forceinline__ void gx_item(const MfArgs &a, const MfTile &tile, int
         // everyone's loads of st + 1 are in; window buffer st % 3 and activation buffer st % 2
         // (read during st - 1) are free
         __syncthreads();
-        if (st + 2 < n_st) issue_x(st + 2);
-        if (st + 3 < n_st) issue_w(st + 3);
+        if constexpr (!SPREAD) {
+#pragma unroll
+            for (int i = 0; i < N_LOADS; i++) issue_next(st, i);
+        }
         if constexpr (NTB > 0) {
             const bool live = 4 * st + grp < nblk;  // past the row's last block
             // the stage read next (unconditionally, so that no register keeps two values: the last
             // stage reads itself again, unused)
             const int sn = more ? st + 1 : st;
+            const uint32_t ob = b_off(sn), oa = a_off(sn), oc = a_off(st);
             i32x8 av[S::NF];
             int sa[S::NF];
 #pragma unroll
             for (int f = 0; f < S::NF; f++) {
-                const uint32_t sh = (aoff(f, st) + 1u) & 3u;
+                // byte s of the five dwords is the block's scale, its codes follow
+                const uint32_t sh = aoff(f, st, oc) & 3u, sel = 0x04030201u + 0x01010101u * sh;
                 // past the row the codes are whatever the window holds: the activations there are
                 // zero and the scale is 1, so the products are 0
-                const i32x4 w4 = {(int)__builtin_amdgcn_alignbyte(ra[f][1], ra[f][0], sh),
-                                  (int)__builtin_amdgcn_alignbyte(ra[f][2], ra[f][1], sh),
-                                  (int)__builtin_amdgcn_alignbyte(ra[f][3], ra[f][2], sh),
-                                  (int)__builtin_amdgcn_alignbyte(ra[f][4], ra[f][3], sh)};
+                const i32x4 w4 = {(int)__builtin_amdgcn_perm(ra[f][1], ra[f][0], sel),
+                                  (int)__builtin_amdgcn_perm(ra[f][2], ra[f][1], sel),
+                                  (int)__builtin_amdgcn_perm(ra[f][3], ra[f][2], sel),
+                                  (int)__builtin_amdgcn_perm(ra[f][4], ra[f][3], sel)};
                 // an FP4 operand is dwords 0..3; the instruction ignores 4..7
                 av[f] = __builtin_shufflevector(w4, w4, 0, 1, 2, 3, -1, -1, -1, -1);
-                sa[f] = (int)(live ? (re[f] & 0xFFu) : 127u);
+                sa[f] = live ? (int)(ra[f][0] >> (8u * sh)) : 127;  // the instruction takes byte 0
             }
+            constexpr int SLOTS = 3 * NB;
 #pragma unroll
             for (int t = 0; t < NTB; t++) {
                 const int sb = bsc[t];
@@ -445,15 +476,22 @@ __device__ __forceinline__ void gx_item(const MfArgs &a, const MfTile &tile, int
                         if (j == 1) acc[f][t] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av[f], bo[t][1], acc[f][t], 4, 2, 0, sa[f], 1, sb);
                         if (j == 2) acc[f][t] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av[f], bo[t][2], acc[f][t], 4, 2, 0, sa[f], 2, sb);
                     }
+                    // a term's operands of st + 1 go into its registers once its MFMAs are issued
+                    // (the scheduling barriers keep the compiler from hoisting the reads, which
+                    // would need a second register set), with this slot's share of the weight
+                    // reads of st + 1 and of the loads
+                    __builtin_amdgcn_sched_barrier(0);
+                    read_b1(t, j, ob);
+                    if (j == 2) read_bs(t, ob);
+                    constexpr int NA_ = S::NF;
+                    const int sl = 3 * t + j;
+#pragma unroll
+                    for (int f = sl * NA_ / SLOTS; f < (sl + 1) * NA_ / SLOTS; f++) read_a1(f, sn, oa);
+#pragma unroll
+                    for (int i = sl * N_LOADS / SLOTS; SPREAD && i < (sl + 1) * N_LOADS / SLOTS; i++) issue_next(st, i);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-                // the block's operands of st + 1 go into its registers once its MFMAs are issued
-                // (the scheduling barrier keeps the compiler from hoisting the reads, which would
-                // need a second register set)
-                __builtin_amdgcn_sched_barrier(0);
-                read_b(t, sn);
             }
-            __builtin_amdgcn_sched_barrier(0);
-            read_a(sn);
         }
     }
 
@@ -574,7 +612,11 @@ __global__ __launch_bounds__(512, 1) void k_gmx(const MfArgs a) {
         if (mt >= n_tiles) continue;  // uniform across the block
         const int nb = b / R;
         __syncthreads();  // every wave is done with the previous item's buffers
-        const MfTile tile = a.tiles[mt];
+        MfTile tile = a.tiles[mt];  // the same for every lane: into scalar registers
+        tile.expert = __builtin_amdgcn_readfirstlane(tile.expert);
+        tile.slot = __builtin_amdgcn_readfirstlane(tile.slot);
+        tile.pos0 = __builtin_amdgcn_readfirstlane(tile.pos0);
+        tile.m = __builtin_amdgcn_readfirstlane(tile.m);
         const int mbs = (tile.m + 15) >> 4, half = wave >> 2, n0 = (mbs + 1) >> 1;
         const int tb0 = half ? n0 : 0, ntb = half ? mbs - n0 : n0;
         switch (ntb) {
