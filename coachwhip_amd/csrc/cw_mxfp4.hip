@@ -232,8 +232,6 @@ __device__ __forceinline__ void gx_item(const MfArgs &a, const MfTile &tile, int
     constexpr int NB = NTB > 0 ? NTB : 1;
     const int grp = lane >> 4, l16 = lane & 15, rg = wave & 3;
     const int nblk = a.k / 32, n_st = (nblk + 3) / 4;
-    uint8_t *const Wb = smem;
-    uint8_t *const Ab = smem + S::WDEPTH * S::W_BYTES;
     const uint32_t Al = lds0 + S::WDEPTH * S::W_BYTES;
 
     const uint8_t *wb0 = a.w0 + (int64_t)tile.slot * a.s0;
