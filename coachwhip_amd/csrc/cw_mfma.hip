@@ -940,7 +940,7 @@ size_t mfma_dense_workspace(int dtype, int64_t m, int64_t n, int64_t k) {
            (S > 1 ? al256((size_t)S * m * n * 4) + al256((size_t)dense_items(dtype, m, n) * 4) : 0);
 }
 
-// Dense Q4_K QMatMul for 2..16 rows of x, one launch after the pack: block b takes weight rows
+// Dense Q4_K QMatMul for 2..16 rows of x, one launch: block b takes weight rows
 // 16b .. 16b+15 over the whole of k, its W waves a share of at most 2 super-blocks each (4 each
 // measured 13.3 against 12.9 us for config 2 at M = 16: half the waves in flight), with all
 // of a wave's loads (the rows' super-block headers and code bytes, and its activation fragments)
@@ -949,18 +949,23 @@ size_t mfma_dense_workspace(int dtype, int64_t m, int64_t n, int64_t k) {
 // activations (lane = token l16, K-group grp), B = a row's 8 codes sc*q (lane = row l16, K-group
 // grp), and the minimum term as a second accumulator with codes -m; each super-block's sums are
 // folded in f32 with the lane's row's d and dmin (a lane's 4 outputs share its row), the waves'
-// partial tiles summed in LDS in wave order, then scaled by the token's activation scale.
+// partial tiles summed in LDS in wave order.
+// X = uint16_t: rows packed by k_pack_f16 with one scale each (xs). X = float: the wave takes its share
+// of x as it is, f32, and gives each token's 256 values of a super-block the power of two that keeps
+// their largest in [2^14, 2^15) of fp16: one launch instead of two, for twice the bytes of x in every
+// block (skinny_f32).
 constexpr int SKINNY_SB = 2;  // super-blocks per wave
-template <int W>
-__global__ __launch_bounds__(64 * W) void k_skinny_q4k(const uint8_t *w, int64_t row_bytes, int n, int k, const uint16_t *x16,
+template <int W, typename X>
+__global__ __launch_bounds__(64 * W) void k_skinny_q4k(const uint8_t *w, int64_t row_bytes, int n, int k, const X *x,
                                                        const float *xs, int m, float *y) {
+    constexpr bool F32 = std::is_same_v<X, float>;
     // a wave's 16 rows x SKINNY_SB super-blocks, copied as 16-byte chunks (row r's bytes at r * RB)
     constexpr int RB = SKINNY_SB * 144, NCH = 16 * RB / 16, NI = (NCH + 63) / 64;
     __shared__ __align__(16) uint8_t wl[W][NI * 1024];
     __shared__ float part[W][16 * 16];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, grp = lane >> 4;
     const int nsb = k / 256, s0 = wave * nsb / W, s1 = (wave + 1) * nsb / W;  // this wave's super-blocks
-    const uint16_t *xr = x16 + (int64_t)min(l16, m - 1) * k + 8 * grp;
+    const X *xr = x + (int64_t)min(l16, m - 1) * k + 8 * grp;
     // every load at once, from clamped rows and super-blocks (those past s1 are not used): the
     // weight bytes as whole 16-byte chunks of each row's run of super-blocks straight into LDS
     // (per-lane 8-byte pieces of 16 rows measured slower), then the activation fragments
@@ -972,14 +977,15 @@ __global__ __launch_bounds__(64 * W) void k_skinny_q4k(const uint8_t *w, int64_t
     }
     uint4 head[SKINNY_SB];
     uint2 qs[SKINNY_SB][4];
-    uint4 xf[SKINNY_SB][8];
+    constexpr int XL = F32 ? 16 : 8;  // 16-byte loads of x per super-block
+    uint4 xl[SKINNY_SB][XL], xf[SKINNY_SB][8];
 #pragma unroll
     for (int j = 0; j < SKINNY_SB; j++) {
         const int sb = min(s0 + j, nsb - 1);
 #pragma unroll
-        for (int kk = 0; kk < 8; kk++) xf[j][kk] = *(const uint4 *)(xr + 256 * sb + 32 * kk);
+        for (int c = 0; c < XL; c++) xl[j][c] = *(const uint4 *)(xr + 256 * sb + (F32 ? 32 * (c >> 1) + 4 * (c & 1) : 32 * c));
     }
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 * SKINNY_SB) : "memory");  // the chunks have landed
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(XL * SKINNY_SB) : "memory");  // the chunks have landed
 #pragma unroll
     for (int j = 0; j < SKINNY_SB; j++) {
         const uint8_t *blk = &wl[wave][l16 * RB + 144 * j];
@@ -993,6 +999,35 @@ __global__ __launch_bounds__(64 * W) void k_skinny_q4k(const uint8_t *w, int64_t
     f32x4 fin = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < SKINNY_SB; j++) {
+        float inv[4] = {1.f, 1.f, 1.f, 1.f};  // 1 / scale of tokens 4*grp + i
+        if constexpr (F32) {
+            float mx = 0.f;
+#pragma unroll
+            for (int c = 0; c < XL; c++) {
+                const float4 f = __builtin_bit_cast(float4, xl[j][c]);
+                mx = fmaxf(mx, fmaxf(fmaxf(fabsf(f.x), fabsf(f.y)), fmaxf(fabsf(f.z), fabsf(f.w))));
+            }
+            mx = fmaxf(mx, __shfl_xor(mx, 16));  // over the token's four K-groups
+            mx = fmaxf(mx, __shfl_xor(mx, 32));
+            int ex = 0;
+            if (mx > 0.f && mx < INFINITY) {
+                frexpf(mx, &ex);
+                ex = min(15 - ex, 126);  // the scale stays finite and its inverse normal
+            }
+            const float sc = ldexpf(1.0f, ex), is = ldexpf(1.0f, -ex);
+#pragma unroll
+            for (int kk = 0; kk < 8; kk++) {
+                const float4 f = __builtin_bit_cast(float4, xl[j][2 * kk]), g = __builtin_bit_cast(float4, xl[j][2 * kk + 1]);
+                const f16x8 h = {(_Float16)(f.x * sc), (_Float16)(f.y * sc), (_Float16)(f.z * sc), (_Float16)(f.w * sc),
+                                 (_Float16)(g.x * sc), (_Float16)(g.y * sc), (_Float16)(g.z * sc), (_Float16)(g.w * sc)};
+                xf[j][kk] = __builtin_bit_cast(uint4, h);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++) inv[i] = __shfl(is, 4 * grp + i);
+        } else {
+#pragma unroll
+            for (int kk = 0; kk < 8; kk++) xf[j][kk] = xl[j][kk];
+        }
         // no branch on the wave's super-block count: a branch here kept the compiler from issuing
         // the later super-blocks' loads before the first one's MFMAs
         f32x4 acc = {0.f, 0.f, 0.f, 0.f}, accm = {0.f, 0.f, 0.f, 0.f};
@@ -1019,7 +1054,7 @@ __global__ __launch_bounds__(64 * W) void k_skinny_q4k(const uint8_t *w, int64_t
         const bool live = s0 + j < s1;
         const float d = live ? h2f(head[j].x & 0xFFFF) : 0.f, dmin = live ? h2f(head[j].x >> 16) : 0.f;
 #pragma unroll
-        for (int i = 0; i < 4; i++) fin[i] += d * acc[i] + dmin * accm[i];
+        for (int i = 0; i < 4; i++) fin[i] += inv[i] * (d * acc[i] + dmin * accm[i]);
     }
     // lane: tokens 4*grp + i of weight row l16
 #pragma unroll
@@ -1030,23 +1065,43 @@ __global__ __launch_bounds__(64 * W) void k_skinny_q4k(const uint8_t *w, int64_t
         float v = 0.f;
 #pragma unroll
         for (int q = 0; q < W; q++) v += part[q][e];
-        if (t < m && r < n) y[(int64_t)t * n + r] = v * xs[t];
+        if (t < m && r < n) y[(int64_t)t * n + r] = F32 ? v : v * xs[t];
     }
 }
 
-// 2..16 rows of Q4_K x: the pack (fp16 activations and their scales), then k_skinny_q4k
+// Where the GEMM takes x as f32 rather than packed by a launch before it (4 blocks, 4 us): one block per
+// CU at most, and at most 128 KB of x per block. us per call, packed / f32: 4096 x 4096 at 2 rows 9.2 / 7.8,
+// at 8 rows 10.3 / 9.2, 4096 x 2048 at 16 rows 8.5 / 7.5, 4096 x 1024 at 16 rows 7.3 / 5.7, 512 x 512 at 16
+// rows 6.6 / 4.8. Past it the loads of x cost as much as the launch or more: 4096 x 4096 at 16 rows 12.1 /
+// 11.8, 4096 x 3072 at 16 rows 10.8 / 11.5, 8192 x 4096 at 2 rows 12.6 / 14.3, at 16 rows 16.3 / 21.4,
+// 5120 x 2048 at 16 rows 10.5 / 11.4. (A 16-wave block, k above 4,096, would not have the registers.)
+static bool skinny_f32(int n, int waves, int m) { return n <= 16 * 256 && m * waves * SKINNY_SB * 256 <= 32768; }
+
+// 2..16 rows of Q4_K x: k_skinny_q4k, after the pack (fp16 activations and their scales) if it takes packed rows
 static int dense_skinny_q4k(const uint8_t *w, int64_t row_bytes, int n, int k, const float *x, int m, float *y, uint16_t *x16,
                             float *xs, hipStream_t s) {
+    const int nsb = k / 256, need = (nsb + SKINNY_SB - 1) / SKINNY_SB;
+    const int waves = need <= 1 ? 1 : need <= 2 ? 2 : need <= 4 ? 4 : need <= 8 ? 8 : 16;
+    if (need > 16) return set_error(CW_ENOTSUP, "qmatmul: k %d above %d for the skinny Q4_K path", k, 16 * SKINNY_SB * 256);
+    const dim3 grid((unsigned)((n + 15) / 16)), block(64 * waves);
+    if (waves <= 8 && skinny_f32(n, waves, m)) {
+#define CW_SKINNY(W) hipLaunchKernelGGL((k_skinny_q4k<W, float>), grid, block, 0, s, w, row_bytes, n, k, x, nullptr, m, y)
+        if (waves == 1) CW_SKINNY(1);
+        else if (waves == 2) CW_SKINNY(2);
+        else if (waves == 4) CW_SKINNY(4);
+        else CW_SKINNY(8);
+#undef CW_SKINNY
+        return check_launch("k_skinny_q4k");
+    }
     int rc;
     if ((rc = pack_rows_f16(x, m, k, k, x16, xs, s, nullptr, K_NATURAL))) return rc;
-    const int nsb = k / 256, waves = (nsb + SKINNY_SB - 1) / SKINNY_SB;
-    const dim3 grid((unsigned)((n + 15) / 16));
-    if (waves <= 1) hipLaunchKernelGGL(k_skinny_q4k<1>, grid, dim3(64), 0, s, w, row_bytes, n, k, x16, xs, m, y);
-    else if (waves <= 2) hipLaunchKernelGGL(k_skinny_q4k<2>, grid, dim3(128), 0, s, w, row_bytes, n, k, x16, xs, m, y);
-    else if (waves <= 4) hipLaunchKernelGGL(k_skinny_q4k<4>, grid, dim3(256), 0, s, w, row_bytes, n, k, x16, xs, m, y);
-    else if (waves <= 8) hipLaunchKernelGGL(k_skinny_q4k<8>, grid, dim3(512), 0, s, w, row_bytes, n, k, x16, xs, m, y);
-    else if (waves <= 16) hipLaunchKernelGGL(k_skinny_q4k<16>, grid, dim3(1024), 0, s, w, row_bytes, n, k, x16, xs, m, y);
-    else return set_error(CW_ENOTSUP, "qmatmul: k %d above %d for the skinny Q4_K path", k, 16 * SKINNY_SB * 256);
+#define CW_SKINNY(W) hipLaunchKernelGGL((k_skinny_q4k<W, uint16_t>), grid, block, 0, s, w, row_bytes, n, k, x16, xs, m, y)
+    if (waves == 1) CW_SKINNY(1);
+    else if (waves == 2) CW_SKINNY(2);
+    else if (waves == 4) CW_SKINNY(4);
+    else if (waves == 8) CW_SKINNY(8);
+    else CW_SKINNY(16);
+#undef CW_SKINNY
     return check_launch("k_skinny_q4k");
 }
 
