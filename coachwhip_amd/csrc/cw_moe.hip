@@ -133,15 +133,17 @@ static bool grouped_path(const cw_moe_desc *d, int T) {
            mfma_supported(d->dtype[2]) && (d->slot_table ? d->n_slots : d->n_experts) <= 1024;
 }
 
-// Layers with a Q5_K or Q6_K matrix have no fp16 GEMM: they run as grouped GEMMs at f32 accuracy (their
-// per-pick matvecs keep f32 activations), where the other formats of the layer can too and every matrix is
-// below the GEMM's 4 GiB, once that is faster. The matvecs read an expert's matrices once per pick
-// (measured about 0.235 us per million weights, + 10 us), the GEMMs once per distinct expert (about 0.245
-// us per million, + 45 us for their launches and rounds), so the GEMMs win where the picks beyond the
-// distinct experts, E (1 - (1 - K / E)^T) on average, come to 150 million weights or more; 230 here, since
-// near the line the matvecs spread better. Measured (matvec / GEMM): Q4_K + Q6_K, 128 experts, top-8, 768
-// x 2048: 16 tokens 136 / 144, 24 tokens 229 / 161; 256 experts of 512: 16 tokens 88 / 128, 24 tokens 150
-// / 149. CWMOE_PREFILL_MIN_TOKENS (tokens) overrides.
+// The grouped GEMMs at f32 accuracy: for layers that keep f32 activations, which are those with a Q5_K or
+// Q6_K matrix (no fp16 GEMM takes them) at any T and those of Q4_K and Q8_0 below prefill_min_tokens, where
+// gate/up and down both are formats of the GEMM and every matrix is below its 4 GiB, once that is faster.
+// The matvecs read an expert's matrices once per pick (measured about 0.235 us per million weights, + 10 us),
+// the GEMMs once per distinct expert (about 0.245 us per million, + 45 us for their launches and rounds), so
+// the GEMMs win where the picks beyond the distinct experts, E (1 - (1 - K / E)^T) on average, come to 150
+// million weights or more; 230 here, since near the line the matvecs spread better. Measured (matvec /
+// GEMM): Q4_K + Q6_K, 128 experts, top-8, 768 x 2048: 16 tokens 136 / 144, 24 tokens 229 / 161; 256 experts
+// of 512: 16 tokens 88 / 128, 24 tokens 150 / 149. Just past the line, 10 tokens: 8 experts, top-2, 2048 x
+// 4096, Q4_K 85.0 / 84.7, Q8_0 98.8 / 90.1; 64 experts, top-8, 1536 x 2048, Q4_K 161 / 126, Q8_0 225 / 161;
+// 15 tokens there 230 / 160 and 317 / 186. CWMOE_PREFILL_MIN_TOKENS (tokens) overrides.
 static bool split_path(const cw_moe_desc *d, int T) {
     if (grouped_path(d, T) || d->dtype[0] != d->dtype[1] || !split_supported(d->dtype[0]) ||
         !split_supported(d->dtype[2]) || (d->slot_table ? d->n_slots : d->n_experts) > 1024)
@@ -725,9 +727,15 @@ int cw_moe_layer_noalloc(const cw_moe_desc *desc, const float *x, const float *l
     return moe_layer(desc, x, logits, T, out, ids_out, w_out, missing, ws, NOALLOC_SCRATCH_BYTES, (hipStream_t)stream);
 }
 
+// Not decreasing in T, so that a workspace (or a captured graph's buffer) of a layer's largest batch serves
+// the smaller ones: the GEMMs of Q4_K and Q8_0 at f32 accuracy, below prefill_min_tokens, may need more than
+// the fp16 GEMMs from there on. A call itself asks for its own layout only.
 size_t cw_moe_workspace_size(const cw_moe_desc *desc, int T) {
     if (check_desc(desc, T)) return 0;
-    return layout(desc, T).total;
+    const int below = prefill_min_tokens() - 1;
+    size_t bytes = layout(desc, T).total;
+    if (below > 0 && grouped_path(desc, T) && split_path(desc, below)) bytes = std::max(bytes, layout(desc, below).total);
+    return bytes;
 }
 
 int cw_moe_layer(const cw_moe_desc *desc, const float *x, const float *logits, int T, float *out, uint32_t *ids_out,

@@ -238,7 +238,12 @@ typedef struct cw_moe_desc {
  * blocks of one-token calls whose barrier gave up or found the state invalid (their outputs are
  * NaN): a caller reads it on its stream (an asynchronous copy after the call), with no device
  * synchronize, and compares it with the value before the call. No counterpart in the reference
- * (its layer is several dispatches). */
+ * (its layer is several dispatches).
+ * From 16 tokens the layer runs as grouped GEMMs on fp16 activations (MXFP4: three FP6 terms). Layers
+ * with a Q5_K or Q6_K matrix, whose other matrices are Q4_K or Q8_0, keep f32 accuracy at every T, as
+ * every layer does below 16 tokens: per-pick matvecs, or, for these formats and as many picks as pay for
+ * it, GEMMs on the activations as two fp16 terms. A workspace that is large enough for the matvecs but
+ * not for those GEMMs is accepted and the matvecs run. cw_moe_workspace_size does not decrease in T. */
 #define CW_MOE_STATE_BYTES 8448
 #define CW_MOE_STATUS_OFFSET 8320
 size_t cw_moe_workspace_size(const cw_moe_desc *desc, int T);
@@ -249,12 +254,13 @@ int cw_moe_layer(const cw_moe_desc *desc, const float *x, const float *logits, i
 /* cw_moe_layer without a workspace, for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid allocation). No counterpart in the
  * reference. Its scratch is one static array per device in the library (CW_MOE_NOALLOC_BYTES,
- * held from the library's load until the process ends); a call whose cw_moe_workspace_size is
- * larger is refused with CW_EINVAL (config 3's shape fits about 90 tokens). The call allocates
- * nothing. Every call on a device shares that device's array: calls that overlap in time on one
- * device (on different streams, or from different threads) race and must not be made. Outputs
- * equal cw_moe_layer's bit for bit (the same kernels; a layer with Q5_K or Q6_K matrices whose GEMMs'
- * workspace does not fit the array takes the per-pick matvecs instead: equal to f32 accuracy). */
+ * held from the library's load until the process ends); a call whose matvecs' or fp16 GEMMs'
+ * workspace is larger is refused with CW_EINVAL (config 3's shape fits about 90 tokens). The call
+ * allocates nothing. Every call on a device shares that device's array: calls that overlap in time
+ * on one device (on different streams, or from different threads) race and must not be made. Outputs
+ * equal cw_moe_layer's bit for bit (the same kernels), but for a call that cw_moe_layer runs as GEMMs
+ * at f32 accuracy (see there) and whose layout of those does not fit the array: it takes the per-pick
+ * matvecs, equal to f32 accuracy. */
 #define CW_MOE_NOALLOC_BYTES ((size_t)8 << 20)
 int cw_moe_layer_noalloc(const cw_moe_desc *desc, const float *x, const float *logits, int T,
                          float *out, uint32_t *ids_out, float *w_out, uint32_t *missing,

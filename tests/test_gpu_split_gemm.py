@@ -1,9 +1,13 @@
 """Q5_K and Q6_K GEMMs at f32 accuracy (activations as two fp16 terms, exact weight codes): dense
 products and MoE layers, against the f64 oracle and the f32 matvec they stand in for."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
+import coachwhip_amd as cw
+from coachwhip_amd import _lib
 from coachwhip_amd import formats as F
 from coachwhip_amd import ops, synth
 from oracle import oracle as O
@@ -85,3 +89,87 @@ def test_layer(pair, tokens, experts, top_k, hidden, inter, monkeypatch):
         err[path] = O.rel_l2(out[path], want)
     assert not np.array_equal(out["gemm"], out["matvec"])
     assert err["gemm"] <= min(2 * REL_L2, 2 * err["matvec"])  # (two products after one another)
+
+
+def _banks(w, experts):
+    shapes = [(w.inter, w.hidden)] * 2 + [(w.hidden, w.inter)]
+    return [ops.ExpertBank.from_blocks(w.host[m], w.dtypes[m], *s, experts) for m, s in enumerate(shapes)]
+
+
+def _call(layer, x, logits, entry="workspace", ws_bytes=None):
+    """cw_moe_layer with a workspace of ws_bytes (what it asks for by default), or the entry point without one."""
+    L, (tokens, hidden) = cw.lib(), x.shape
+    out = torch.empty((tokens, hidden), device="cuda")
+    p = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    if entry == "noalloc":
+        _lib.check(L.cw_moe_layer_noalloc(ctypes.byref(layer.desc), p(x), p(logits), tokens, p(out), None, None, None, None))
+    else:
+        need = L.cw_moe_workspace_size(ctypes.byref(layer.desc), tokens) if ws_bytes is None else ws_bytes
+        ws = torch.zeros(need, dtype=torch.uint8, device="cuda")
+        _lib.check(L.cw_moe_layer(ctypes.byref(layer.desc), p(x), p(logits), tokens, p(out), None, None, None, p(ws), need, None))
+    torch.cuda.synchronize()
+    return out.cpu().numpy()
+
+
+# no override: every token picks all four experts, 264 million weights beyond the distinct ones at 15 tokens
+# and 246 million at 14 of the second shape
+@pytest.mark.parametrize("pair", [(F.Q4_K, F.Q4_K), (F.Q8_0, F.Q8_0), (F.Q4_K, F.Q8_0), (F.Q4_K, F.Q6_K)],
+                         ids=lambda p: F.NAMES[p[0]] + "-" + F.NAMES[p[1]])
+@pytest.mark.parametrize("tokens,hidden,inter", [(15, 1024, 1536), (14, 2048, 768)])
+def test_layer_by_the_rule_and_with_less_workspace(pair, tokens, hidden, inter, monkeypatch):
+    monkeypatch.delenv("CWMOE_PREFILL_MIN_TOKENS", raising=False)
+    rng = np.random.default_rng(tokens + inter)
+    w = synth.moe_weights(4, 4, hidden, inter, (pair[0],) + pair, rng)
+    layer = ops.MoeLayer(*_banks(w, 4), n_experts=4, top_k=4)
+    x, logits = rng.standard_normal((tokens, hidden)).astype(np.float32), rng.standard_normal((tokens, 4)).astype(np.float32)
+    want = O.moe_layer(w, x, logits)[0]
+    x, logits = ops.to_device(x), ops.to_device(logits)
+    gemm, noalloc = _call(layer, x, logits), _call(layer, x, logits, "noalloc")
+    matvec = cw.lib().cw_moe_workspace_size(ctypes.byref(layer.desc), 4)  # below the line: the matvecs' layout
+    matvec += 3 * 1024 + (tokens - 4) * 4 * 4 * inter                    # for all tokens
+    less = _call(layer, x, logits, ws_bytes=matvec)
+    monkeypatch.setenv("CWMOE_PREFILL_MIN_TOKENS", "1000000")
+    plain = _call(layer, x, logits)
+    assert np.array_equal(gemm.view(np.uint32), noalloc.view(np.uint32))  # the GEMMs' layout fits its array
+    assert np.array_equal(less.view(np.uint32), plain.view(np.uint32)) and not np.array_equal(gemm, plain)
+    assert O.rel_l2(gemm, want) <= min(2 * REL_L2, 2 * O.rel_l2(plain, want))
+
+
+def test_noalloc_layer_whose_gemms_do_not_fit(monkeypatch):
+    """110 tokens of 8 picks: 2.2 MB for the matvecs, 15 MB for the GEMMs."""
+    monkeypatch.delenv("CWMOE_PREFILL_MIN_TOKENS", raising=False)
+    rng = np.random.default_rng(9)
+    w = synth.moe_weights(8, 8, 2816, 512, (F.Q4_K, F.Q4_K, F.Q6_K), rng)
+    layer = ops.MoeLayer(*_banks(w, 8), n_experts=8, top_k=8)
+    x, logits = rng.standard_normal((110, 2816)).astype(np.float32), rng.standard_normal((110, 8)).astype(np.float32)
+    want = O.moe_layer(w, x, logits)[0]
+    x, logits = ops.to_device(x), ops.to_device(logits)
+    assert cw.lib().cw_moe_workspace_size(ctypes.byref(layer.desc), 110) > 8 << 20
+    gemm, noalloc = _call(layer, x, logits), _call(layer, x, logits, "noalloc")
+    assert not np.array_equal(gemm, noalloc)
+    for got in (gemm, noalloc):
+        assert O.rel_l2(got, want) <= 2 * REL_L2
+
+
+@pytest.mark.parametrize("dtype", [F.Q5_K, F.Q6_K])
+def test_dense_by_the_rule_and_without_workspace(dtype, monkeypatch):
+    monkeypatch.delenv("CWMOE_MM_MIN_ROWS", raising=False)
+    rng = np.random.default_rng(dtype)
+    n, k, m = 640, 2048, 40  # 248 million of 215 needed
+    raw = synth.random_blocks(dtype, n * k, rng)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    want = O.qmatmul_f64(dtype, raw, n, k, x)
+    L, w, xd = cw.lib(), ops.to_device(raw), ops.to_device(x)
+    p = lambda t: None if t is None else ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    need, got = L.cw_qmatmul_workspace_size(dtype, n, k, m), {}
+    assert need > 0
+    for name, size in (("gemm", need), ("short", need - 1), ("none", 0)):
+        ws = torch.empty(size, dtype=torch.uint8, device="cuda") if size else None
+        y = torch.empty((m, n), device="cuda")
+        _lib.check(L.cw_qmatmul(dtype, p(w), n, k, p(xd), m, p(y), p(ws), size, None))
+        torch.cuda.synchronize()
+        got[name] = y.cpu().numpy()
+    monkeypatch.setenv("CWMOE_MM_MIN_ROWS", "1000000")
+    plain = ops.QMatMul(ops.QTensor.from_blocks(raw, dtype, (n, k))).forward(xd).cpu().numpy()
+    assert np.array_equal(got["short"], plain) and np.array_equal(got["none"], plain) and not np.array_equal(got["gemm"], plain)
+    assert O.rel_l2(got["gemm"], want) <= min(REL_L2, 2 * O.rel_l2(plain, want))
