@@ -110,9 +110,10 @@ int combine_picks(const float *dn, const float *w, const float *bias, const uint
                   int T, int K, int H, float *out, hipStream_t s);
 
 // The same GEMMs at f32 accuracy (cw_mfma_split.hip): activations as two fp16 terms, exact weight codes.
-// Rows of split_row halves, packed for the weights' format.
+// Rows of split_row halves, packed for the weights' format, with split_scales scales each.
 bool split_supported(int dtype);
 int split_row(int dtype, int64_t k);
+int split_scales(int64_t k);
 int pack_rows_split(int dtype, const float *x, int rows, int k, int ldx, uint16_t *a16, float *ascale, hipStream_t s,
                     const PackExtra *extra = nullptr);
 int split_gateup(int dtype, const MfArgs &a, int tiles_max, hipStream_t s);

@@ -1,16 +1,21 @@
 // Grouped and dense GEMMs at f32 accuracy on the fp16 matrix instruction (gfx950), for the formats whose
 // other path is one f32 matvec per row of x: Q5_K and Q6_K, and the formats they share a layer with.
 //
-// Every activation goes in as two fp16 terms of one power-of-two row scale, hi = fp16(x) and lo =
-// fp16(x - hi), which together hold x to 2^-23 of itself (terms below 2^-24 of fp16's unit, 2^-39 of the
-// row's largest value, vanish). The weight codes are integers that fp16 holds exactly: sc * q of Q4_K
-// (at most 945) and Q5_K (at most 1,953), Q8_0's quants; Q6_K's sc * (q - 32) reaches
-// 4,096 and goes in as its fp16 rounding and the exact rest (0 or +-1). A product then is two matrix
-// instructions per fragment (three for Q6_K, whose rest times lo is below 2^-23 of the product), each
-// product exact in the f32 accumulators. The minimum term of Q4_K and Q5_K is a ninth K-step per
-// super-block: codes m against the sub-blocks' sums of x (computed in f32 by the pack, two fp16 terms).
-// A super-block's sum is scaled into a second accumulator set in f32, so no running scale's rounding is
-// carried through a row.
+// Every activation goes in as two fp16 terms under a power of two per super-block of its row, hi = fp16(x)
+// and lo = fp16((x - hi) 2^12), which together hold x to 2^-23 of itself, and values below 2^-29 of the
+// super-block's largest to 2^-52 of that. The weight codes are numbers that fp16 holds exactly: sc (q - C) / 2
+// of Q4_K and Q5_K (C the middle of q's range), Q8_0's quants; Q6_K's sc (q - 32) reaches 4,096 and goes
+// in as its fp16 rounding and the exact rest (0 or +-1). A product then is two matrix instructions per
+// fragment (three for Q6_K, whose rest times lo is below 2^-23 of the product), hi and what is below it in
+// accumulators of their own: an instruction rounds its accumulator every 8 products, at the size of its sums,
+// so the small terms cost the large ones nothing. The minimum term of Q4_K and Q5_K and what C took off are a
+// ninth K-step per super-block: codes m and C sc against the sub-blocks' sums of x, which the pack takes in
+// f64 and holds in three terms, so that what all weights of a sub-block have in common meets x exactly.
+// A super-block's sum is scaled into a further accumulator set in f32, so no running scale's rounding is
+// carried through a row. Error against f64 (rel-L2; the matvec's, then with one scale and one accumulator per
+// row and uncentred codes): Q5_K 513 x 4096 at 77 rows 1.08e-7 (1.35, 1.75), Q6_K 1.35e-7 (2.15, 1.69); layers
+// of 4 experts, 15 tokens, 4096 x 512: Q8_0 / Q4_K 2.1e-7 (2.4, 8.0), Q4_K / Q8_0 2.1e-7 (2.3, 3.0), Q5_K /
+// Q6_K 2.1e-7 (3.9, 3.1), Q4_K alone 0.9e-7 (0.8, 1.2).
 #include <math.h>
 
 #include <atomic>
@@ -24,88 +29,82 @@ namespace cw {
 
 // ------------------------------------------------------------------------------ formats
 // Per format: NF code fragments per K-step of 32 weights (lane group grp: weights 8 grp .. 8 grp + 7),
-// MIN the minimum step, STEP a scale per K-step instead of one per super-block (stage). Stage holds
+// MIN the step of the sums, STEP a scale per K-step instead of one per super-block (stage). Stage holds
 // what a lane needs of its row for the whole stage; w is the row's window from the stage's first byte.
 
-__device__ __forceinline__ uint4 codes_exact(uint32_t q0, uint32_t q1, float sc) {  // sc * q, q < 64
-    return fma4(bytes_plus_1024(q0, q1), splat_f16f(sc), splat_f16f(-1024.0f * sc));
+// the terms' second halves are held times LO (k_pack_split)
+constexpr float LO = 4096.0f;
+constexpr uint32_t LO_F16X2 = 0x6C006C00u, LO_INV_F16X2 = 0x0C000C00u;  // LO and 1 / LO, twice each
+
+// half i of an fp16 pair, twice (an operand select of the packed instruction that takes it)
+__device__ __forceinline__ uint32_t splat_half(uint32_t v, int i) {
+    const f16x2 h = __builtin_bit_cast(f16x2, v);
+    return __builtin_bit_cast(uint32_t, f16x2{h[i], h[i]});
 }
-// scale and minimum of sub-block j from the 12 scale bytes of a Q4_K or Q5_K super-block (j a constant)
-__device__ __forceinline__ void k4_const(const uint32_t (&b)[3], int j, uint32_t &sc, uint32_t &m) {
-    const int sh = 8 * (j & 3);
-    if (j < 4) {
-        sc = (b[0] >> sh) & 63;
-        m = (b[1] >> sh) & 63;
-    } else {
-        sc = ((b[2] >> sh) & 0xF) | (((b[0] >> (sh + 6)) & 3) << 4);
-        m = ((b[2] >> (sh + 4)) & 0xF) | (((b[1] >> (sh + 6)) & 3) << 4);
+// sc (q - C) / 2 for q < 64, from s2 = sc / 2 twice: the bytes q + 64 - C under 0x64 are 1088 + q - C, and
+// 544 sc is exact in fp16 (17 times a 6-bit number), as is every code (at most 10 bits and a half)
+template <int C>
+__device__ __forceinline__ uint4 codes_centred(uint32_t q0, uint32_t q1, uint32_t s2) {
+    constexpr uint32_t off = 0x01010101u * (64 - C);
+    return fma4(bytes_plus_1024(q0 + off, q1 + off), s2, pk_mul_u(s2, 0xE440E440u));  // -1088
+}
+// What Q4_K and Q5_K share: d, dmin and the 12 bytes of eight 6-bit scales and minima (get_scale_min_k4)
+struct K4Stage {
+    uint32_t s2[4];  // half of the scales of sub-blocks 2i and 2i + 1, fp16
+    __device__ __forceinline__ void load_scales(const WinRef &w) {
+        const uint32_t b0 = w.u32(4), b2 = w.u32(12);
+        const uint4 x = fma4(bytes_plus_1024(b0 & 0x3F3F3F3Fu, (b2 & 0x0F0F0F0Fu) | ((b0 >> 2) & 0x30303030u)), 0x38003800u, 0xE000E000u);  // (x - 1024) / 2
+        s2[0] = x.x;
+        s2[1] = x.y;
+        s2[2] = x.z;
+        s2[3] = x.w;
     }
-}
-__device__ __forceinline__ uint4 k4_mins(const uint32_t (&b)[3]) {  // the 8 minima as fp16
-    uint32_t o[4];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        uint32_t s, m0, m1;
-        k4_const(b, 2 * i, s, m0);
-        k4_const(b, 2 * i + 1, s, m1);
-        o[i] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz((float)m0, (float)m1));
+    // the codes that meet the sub-blocks' sums of x over 32, times one: the minima, and the scales' halves
+    // times 32 C for what the centre took off the codes
+    template <int C>
+    __device__ __forceinline__ void sums_codes(const WinRef &w, float one, f16x8 &mins, f16x8 &scs) const {
+        const uint32_t b1 = w.u32(8), b2 = w.u32(12), f = splat_f16f(32.f * C * one);
+        mins = as_f16x8(fma4(bytes_plus_1024(b1 & 0x3F3F3F3Fu, ((b2 >> 4) & 0x0F0F0F0Fu) | ((b1 >> 2) & 0x30303030u)), splat_f16f(one),
+                             splat_f16f(-1024.f * one)));
+        scs = as_f16x8(scale4(make_uint4(s2[0], s2[1], s2[2], s2[3]), f));
     }
-    return make_uint4(o[0], o[1], o[2], o[3]);
-}
+    // d for codes that are halves, dmin for sums over 32
+    static __device__ __forceinline__ void scales(const WinRef &w, float &d, float &dm) {
+        const uint32_t dd = w.u32(0);
+        d = 2.f * h2f(dd & 0xFFFFu);
+        dm = -32.f * h2f(dd >> 16);
+    }
+};
 
 struct SQ4_K {
-    static constexpr int TS = 144, SBK = 256, NF = 1;
+    static constexpr int TS = 144, SBK = 256, NF = 1, C = 8;
     static constexpr bool MIN = true, STEP = false;
-    struct Stage {
-        uint32_t b[3];
-        float d, dm;
-        __device__ __forceinline__ void load(const WinRef &w, int) {
-            const uint32_t dd = w.u32(0);
-            const uint2 lo = w.u64(4);
-            b[0] = lo.x;
-            b[1] = lo.y;
-            b[2] = w.u32(12);
-            d = h2f(dd & 0xFFFFu);
-            dm = h2f(dd >> 16);
-        }
-        __device__ __forceinline__ uint4 mins() const { return k4_mins(b); }
+    struct Stage : K4Stage {
+        __device__ __forceinline__ void load(const WinRef &w, int) { load_scales(w); }
     };
     static __device__ __forceinline__ float make(const WinRef &w, const Stage &st, int kk, int grp, uint4 (&f)[1]) {
-        uint32_t sc, m;
-        k4_const(st.b, kk, sc, m);
         const uint2 q = w.u64(16 + 32 * (kk >> 1) + 8 * grp);
         const int sh = 4 * (kk & 1);
-        f[0] = codes_exact((q.x >> sh) & 0x0F0F0F0Fu, (q.y >> sh) & 0x0F0F0F0Fu, (float)sc);
+        f[0] = codes_centred<C>((q.x >> sh) & 0x0F0F0F0Fu, (q.y >> sh) & 0x0F0F0F0Fu, splat_half(st.s2[kk >> 1], kk & 1));
         return 0.f;
     }
 };
 
 struct SQ5_K {
-    static constexpr int TS = 176, SBK = 256, NF = 1;
+    static constexpr int TS = 176, SBK = 256, NF = 1, C = 16;
     static constexpr bool MIN = true, STEP = false;
-    struct Stage {
-        uint32_t b[3];
+    struct Stage : K4Stage {
         uint2 h;  // the lane's bytes of qh: bit kk is weight kk's fifth
-        float d, dm;
         __device__ __forceinline__ void load(const WinRef &w, int grp) {
-            const uint32_t dd = w.u32(0);
-            const uint2 lo = w.u64(4);
-            b[0] = lo.x;
-            b[1] = lo.y;
-            b[2] = w.u32(12);
+            load_scales(w);
             h = w.u64(16 + 8 * grp);
-            d = h2f(dd & 0xFFFFu);
-            dm = h2f(dd >> 16);
         }
-        __device__ __forceinline__ uint4 mins() const { return k4_mins(b); }
     };
     static __device__ __forceinline__ float make(const WinRef &w, const Stage &st, int kk, int grp, uint4 (&f)[1]) {
-        uint32_t sc, m;
-        k4_const(st.b, kk, sc, m);
         const uint2 q = w.u64(48 + 32 * (kk >> 1) + 8 * grp);
         const int sh = 4 * (kk & 1);
-        f[0] = codes_exact(((q.x >> sh) & 0x0F0F0F0Fu) | (((st.h.x >> kk) & 0x01010101u) << 4),
-                           ((q.y >> sh) & 0x0F0F0F0Fu) | (((st.h.y >> kk) & 0x01010101u) << 4), (float)sc);
+        f[0] = codes_centred<C>(((q.x >> sh) & 0x0F0F0F0Fu) | (((st.h.x >> kk) & 0x01010101u) << 4),
+                                ((q.y >> sh) & 0x0F0F0F0Fu) | (((st.h.y >> kk) & 0x01010101u) << 4), splat_half(st.s2[kk >> 1], kk & 1));
         return 0.f;
     }
 };
@@ -114,31 +113,32 @@ struct SQ6_K {
     static constexpr int TS = 210, SBK = 256, NF = 2;
     static constexpr bool MIN = false, STEP = false;
     struct Stage {
-        uint32_t sc[4];  // the lane's half of each K-step: at bit 16 (kk & 1) of sc[kk >> 1]
-        float d, dm;
+        uint32_t sc[4];  // the scales of the lane's half of K-steps 2i and 2i + 1, fp16
         __device__ __forceinline__ void load(const WinRef &w, int grp) {
             const uint2 a = w.u64(192), b = w.u64(200);
             const int sh = 8 * (grp >> 1);
-            sc[0] = a.x >> sh;
-            sc[1] = a.y >> sh;
-            sc[2] = b.x >> sh;
-            sc[3] = b.y >> sh;
-            d = h2f(w.u32(208) & 0xFFFFu);
+            const uint32_t v[4] = {a.x, a.y, b.x, b.y};
+#pragma unroll
+            for (int i = 0; i < 4; i++)  // (s + 128) + 1024, less 1152
+                sc[i] = pk_fma_u((((v[i] >> sh) & 0x00FF00FFu) ^ 0x00800080u) | 0x64006400u, 0x3C003C00u, 0xE480E480u);
         }
-        __device__ __forceinline__ uint4 mins() const { return make_uint4(0, 0, 0, 0); }
     };
+    static __device__ __forceinline__ float scale(const WinRef &w) { return h2f(w.u32(208) & 0xFFFFu); }
     static __device__ __forceinline__ float make(const WinRef &w, const Stage &st, int kk, int grp, uint4 (&f)[2]) {
         const int h = kk >> 2, r = kk & 3;
         const uint2 l = w.u64(64 * h + 32 * (r & 1) + 8 * grp), g = w.u64(128 + 32 * h + 8 * grp);
         const int sh = 4 * (r >> 1);
         const uint32_t q0 = ((l.x >> sh) & 0x0F0F0F0Fu) | (((g.x >> (2 * r)) & 0x03030303u) << 4);
         const uint32_t q1 = ((l.y >> sh) & 0x0F0F0F0Fu) | (((g.y >> (2 * r)) & 0x03030303u) << 4);
-        const uint32_t sc = splat_f16f((float)(int8_t)(st.sc[kk >> 1] >> (16 * (kk & 1))));
+        const uint32_t sc = splat_half(st.sc[kk >> 1], kk & 1);
         const uint4 c = fma4(bytes_plus_1024(q0, q1), 0x3C003C00u, 0xE420E420u);  // 1.0, -1056.0: q - 32
         f[0] = scale4(c, sc);
-        // the rest of the product: c sc - fp16(c sc), exact
-        const uint4 n = make_uint4(f[0].x ^ 0x80008000u, f[0].y ^ 0x80008000u, f[0].z ^ 0x80008000u, f[0].w ^ 0x80008000u);
-        f[1] = make_uint4(pk_fma_u(c.x, sc, n.x), pk_fma_u(c.y, sc, n.y), pk_fma_u(c.z, sc, n.z), pk_fma_u(c.w, sc, n.w));
+        // the rest of the product, c sc - fp16(c sc), exact, 0 or +-1; times LO, beside the lo terms
+        auto rest = [&](uint32_t x, uint32_t p) __attribute__((always_inline)) {
+            const f16x2 n = -__builtin_bit_cast(f16x2, p);
+            return pk_mul_u(pk_fma_u(x, sc, __builtin_bit_cast(uint32_t, n)), LO_F16X2);
+        };
+        f[1] = make_uint4(rest(c.x, f[0].x), rest(c.y, f[0].y), rest(c.z, f[0].z), rest(c.w, f[0].w));
         return 0.f;
     }
 };
@@ -147,10 +147,9 @@ struct SQ8_0 {
     static constexpr int TS = 34, SBK = 32, NF = 1;
     static constexpr bool MIN = false, STEP = true;
     struct Stage {
-        float d, dm;
         __device__ __forceinline__ void load(const WinRef &, int) {}
-        __device__ __forceinline__ uint4 mins() const { return make_uint4(0, 0, 0, 0); }
     };
+    static __device__ __forceinline__ float scale(const WinRef &) { return 1.f; }
     static __device__ __forceinline__ float make(const WinRef &w, const Stage &, int kk, int grp, uint4 (&f)[1]) {
         const uint2 q = w.u64x(TS * kk + 2 + 8 * grp);
         f[0] = fma4(bytes_plus_1024(q.x ^ 0x80808080u, q.y ^ 0x80808080u), 0x3C003C00u, 0xE480E480u);  // 1.0, -1152.0
@@ -165,8 +164,11 @@ struct SQ8_0 {
 // activations in parts of KA K-steps, both terms, through two buffers: a part loads while the one before
 // it is computed. Two blocks share a CU, so one's waits fall into the other's K-steps: with one window
 // buffer a stage starts with a round trip to memory, and that is what bounds it. Against a matvec per row
-// or pick: Q6_K 4001 x 4096 at 77 rows 215 -> 33 us (pack included), error against f64 2.1e-7 -> 1.7e-7; a
-// layer of 128 experts, top-8, Q4_K 768 x 2048 and Q6_K 2048 x 768 at 301 tokens 2.3 ms -> about 0.25.
+// or pick: Q6_K 4001 x 4096 at 77 rows 215 -> 34 us (pack included); a layer of 128 experts, top-8, Q4_K 768 x
+// 2048 and Q6_K 2048 x 768 at 301 tokens 2.3 ms -> 0.22. What the small terms' own accumulators, the centred
+// codes and the scales per super-block cost: nothing at few rows (Q5_K 4096 x 4096 at 77 rows 35 -> 34 us, the
+// pack no longer one wave per row, and the 6-bit scales unpacked once per stage), 2 to 5 % at full tiles (Q6_K
+// 4096 x 4096 at 512 rows 81 -> 84, a layer of 64 experts, Q5_K and Q6_K, 700 tokens 274 -> 288).
 template <class SF, int MODE>
 struct SpShape {
     static constexpr int KST = 8, NW = 8, NT = 64 * NW, NM = MODE == 0 ? 2 : 1, WPM = NW / NM, RPB = 16 * WPM;
@@ -175,7 +177,7 @@ struct SpShape {
     static constexpr int W_BYTES = NM * RPB * WB;
     static constexpr int KA = 2, PARTS = KST / KA + (SF::MIN ? 1 : 0);
     static constexpr int PART = KA * 2 * MF_MB * 1024, A_BYTES = 2 * PART;
-    static constexpr int META = MF_MT * 8, PER_CU = 2;
+    static constexpr int META = 2 * 128 * 4 + MF_MT * 4, PER_CU = 2;  // a stage's scales and the activation rows (by whole waves), picks
     static constexpr size_t lds_bytes() { return W_BYTES + A_BYTES + META; }
     static_assert(PER_CU * (W_BYTES + A_BYTES + META) <= 160 * 1024, "two blocks per CU");
     static_assert(MF_MT * RPB * 4 <= A_BYTES, "the gate/up exchange fits the activation buffers");
@@ -191,7 +193,7 @@ __global__ __launch_bounds__(512, 4) void k_gms(const MfArgs a) {
     __shared__ int split_last;
     uint8_t *As = smem, *Ws = smem + S::A_BYTES;
     float *meta_sa = (float *)(Ws + S::W_BYTES);
-    int *meta_pick = (int *)(meta_sa + MF_MT);
+    int *meta_row = (int *)(meta_sa + 128), *meta_pick = meta_row + 128;
     const int n_nb = (a.n + S::RPB - 1) / S::RPB, R = a.run_tiles, n_tiles = *a.n_tiles;
     const int n_ks = a.k / 32, n_st = (n_ks + KST - 1) / KST;
     const int st_lo = a.split_st ? blockIdx.y * a.split_st : 0, st_hi = a.split_st ? min(n_st, st_lo + a.split_st) : n_st;
@@ -207,10 +209,12 @@ __global__ __launch_bounds__(512, 4) void k_gms(const MfArgs a) {
         const int mw = S::NM > 1 ? wave / S::WPM : 0, wrow = (wave - mw * S::WPM) * 16;  // this wave's matrix and its first row there
         const MfTile tile = a.tiles[mt];
         const int mbs = (tile.m + 15) >> 4;
-        if (tid < tile.m) {  // (the first stage's barriers publish these)
-            const int pos = tile.pos0 + tid;
-            meta_sa[tid] = a.ascale[a.rows ? a.rows[pos] : pos];
-            meta_pick[tid] = a.pile_pick ? a.pile_pick[pos] : pos;
+        if (tid < tile.m) meta_pick[tid] = a.pile_pick ? a.pile_pick[tile.pos0 + tid] : tile.pos0 + tid;  // (the first stage's barriers publish it)
+        // the first two waves bring a stage's scales, one per row of the tile (rows past the last: that one's; a
+        // lane reads back its own)
+        if (wave < 2) {
+            const int pos = tile.pos0 + min(tid, tile.m - 1);
+            meta_row[tid] = a.rows ? a.rows[pos] : pos;
         }
         // the activation row that this lane copies (pick block `wave`): hi at 0, lo at k, the sums at 2 k
         const bool stager = wave < mbs;
@@ -222,7 +226,7 @@ __global__ __launch_bounds__(512, 4) void k_gms(const MfArgs a) {
             const int n = nblk * S::RPB + (r - m * S::RPB);
             return (uint32_t)(n < a.n ? n : 0) * (uint32_t)a.row_bytes;
         };
-        const uint32_t as_lds = lds_addr(As), ws_lds = lds_addr(Ws);
+        const uint32_t as_lds = lds_addr(As), ws_lds = lds_addr(Ws), sa_lds = lds_addr(meta_sa);
         // windows as in k_gmm: each piece's row and place once per tile, 32-bit offsets from the 16-byte
         // boundary below the matrix
         constexpr int NP = S::NM * S::RPB * S::PCS, NTW = (NP + S::NT - 1) / S::NT;
@@ -240,6 +244,7 @@ __global__ __launch_bounds__(512, 4) void k_gms(const MfArgs a) {
             if constexpr (ALIGNED) wp_off[t] = (wp_off[t] & ~15u) + 16 * min(wp_p[t], ((m == 0 ? b0 : b1) + S::SEG - 1) >> 4);
         }
         auto issue_w = [&](int st) __attribute__((always_inline)) {
+            if (wave < 2) dma4(a.ascale + (int64_t)meta_row[tid] * n_st + st, sa_lds + 256 * wave);
             const uint32_t seg = SF::SBK == 32 ? SF::TS * min(KST, n_ks - st * KST) : SF::TS, at = (uint32_t)(S::SEG * st);
 #pragma unroll
             for (int t = 0; t < NTW; t++) {
@@ -281,10 +286,12 @@ __global__ __launch_bounds__(512, 4) void k_gms(const MfArgs a) {
                 const int nk = min(KST, n_ks - st * KST);
                 const WinRef w = WinRef::at<0>(Ws + (mw * S::RPB + wrow + l16) * S::WB + ((lmis + (uint32_t)(S::SEG * st)) & 15));
                 typename SF::Stage stg;
-                f32x4 acc[MBS];
+                // hi times the codes, and (over LO) what is below it: lo times the codes and hi times Q6_K's rest.
+                // With a scale per K-step: the stage's sum of both, scaled
+                f32x4 acc[MBS], low[MBS];
 #pragma unroll
                 for (int p = 0; p < S::PARTS; p++) {
-                    __builtin_amdgcn_s_waitcnt(0);  // this part's activations (and the windows)
+                    __builtin_amdgcn_s_waitcnt(0);  // this part's activations (and the windows and scales)
                     __syncthreads();
                     if (p + 1 < S::PARTS) issue_a(st, p + 1, buf ^ 1);
                     else if (st + 1 < st_hi) issue_a(st + 1, 0, buf ^ 1);
@@ -292,16 +299,24 @@ __global__ __launch_bounds__(512, 4) void k_gms(const MfArgs a) {
                     auto av = [&](int step, int term, int mb) __attribute__((always_inline)) {
                         return *(const f16x8 *)(A + ((2 * step + term) * MF_MB + mb) * 1024);
                     };
+                    // the scales of this lane's rows, 16 mb + 4 grp ..
+                    auto sa = [&](int mb) __attribute__((always_inline)) { return *(const f32x4 *)(meta_sa + 16 * mb + 4 * grp); };
                     buf ^= 1;
                     if (p == 0) stg.load(w, grp);
-                    if (SF::MIN && p == KST / KA) {
-                        const f16x8 m = as_f16x8(stg.mins());
-                        const float sc = -32.f * stg.dm;  // (the sums are held over 32)
+                    if constexpr (SF::MIN) if (p == KST / KA) {
+                        // K positions 0..7 the sums' hi, 8..23 what is below it (times LO), then zeros
+                        f16x8 fm, fs;
+                        float d, dm;
+                        stg.template sums_codes<SF::C>(w, grp == 0 ? 1.f : 1.f / LO, fm, fs);
+                        stg.scales(w, d, dm);
 #pragma unroll
                         for (int mb = 0; mb < MBS; mb++) {
-                            const f32x4 c = __builtin_amdgcn_mfma_f32_16x16x32_f16(av(0, 0, mb), m, f32x4{0, 0, 0, 0}, 0, 0, 0);
+                            const f16x8 sums = av(0, 0, mb);
+                            const f32x4 c = __builtin_amdgcn_mfma_f32_16x16x32_f16(sums, fm, f32x4{0, 0, 0, 0}, 0, 0, 0), s = sa(mb);
+                            acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(sums, fs, acc[mb], 0, 0, 0);
 #pragma unroll
-                            for (int i = 0; i < 4; i++) tot[mb][i] = fmaf(c[i], sc, tot[mb][i]);
+                            for (int i = 0; i < 4; i++)
+                                tot[mb][i] = fmaf(fmaf(c[i], dm, fmaf(low[mb][i], 1.f / LO, acc[mb][i]) * d), s[i], tot[mb][i]);
                         }
                         continue;
                     }
@@ -314,23 +329,32 @@ __global__ __launch_bounds__(512, 4) void k_gms(const MfArgs a) {
 #pragma unroll
                         for (int mb = 0; mb < MBS; mb++) {
                             const f16x8 hi = av(q, 0, mb), lo = av(q, 1, mb);
-                            f32x4 c = SF::STEP || kk == 0 ? f32x4{0, 0, 0, 0} : acc[mb];
-                            c = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo, as_f16x8(f[0]), c, 0, 0, 0);
-                            if constexpr (SF::NF > 1) c = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, as_f16x8(f[1]), c, 0, 0, 0);
+                            const f32x4 z = {0, 0, 0, 0};
+                            f32x4 c = SF::STEP || kk == 0 ? z : acc[mb], l = SF::STEP || kk == 0 ? z : low[mb];
+                            l = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo, as_f16x8(f[0]), l, 0, 0, 0);
                             c = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, as_f16x8(f[0]), c, 0, 0, 0);
-                            acc[mb] = c;
+                            if constexpr (SF::NF > 1) l = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, as_f16x8(f[1]), l, 0, 0, 0);
                             if constexpr (SF::STEP) {
 #pragma unroll
-                                for (int i = 0; i < 4; i++) tot[mb][i] = fmaf(c[i], sd, tot[mb][i]);
+                                for (int i = 0; i < 4; i++) acc[mb][i] = fmaf(fmaf(l[i], 1.f / LO, c[i]), sd, kk == 0 ? 0.f : acc[mb][i]);
+                            } else {
+                                acc[mb] = c;
+                                low[mb] = l;
                             }
                         }
                         __builtin_amdgcn_sched_barrier(0);  // (the steps interleaved run out of registers)
                     }
-                    if (!SF::STEP && p == KST / KA - 1) {
+                    if constexpr (!SF::MIN) if (p == KST / KA - 1) {
+                        const float d = SF::scale(w);
 #pragma unroll
-                        for (int mb = 0; mb < MBS; mb++)
+                        for (int mb = 0; mb < MBS; mb++) {
+                            const f32x4 s = sa(mb);
 #pragma unroll
-                            for (int i = 0; i < 4; i++) tot[mb][i] = fmaf(acc[mb][i], stg.d, tot[mb][i]);
+                            for (int i = 0; i < 4; i++) {
+                                if constexpr (SF::STEP) tot[mb][i] = fmaf(acc[mb][i], s[i], tot[mb][i]);
+                                else tot[mb][i] = fmaf(fmaf(low[mb][i], 1.f / LO, acc[mb][i]) * s[i], d, tot[mb][i]);
+                            }
+                        }
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
@@ -356,7 +380,7 @@ __global__ __launch_bounds__(512, 4) void k_gms(const MfArgs a) {
 #pragma unroll
                 for (int i = 0; i < 2; i++) {
                     const int r = 16 * mb + 4 * grp + (mw == 0 ? 2 : 0) + i;
-                    xv[r * S::RPB + wrow + l16] = (mw == 0 ? tot[mb][2 + i] : tot[mb][i]) * meta_sa[r];
+                    xv[r * S::RPB + wrow + l16] = mw == 0 ? tot[mb][2 + i] : tot[mb][i];
                 }
             }
             __syncthreads();
@@ -368,7 +392,7 @@ __global__ __launch_bounds__(512, 4) void k_gms(const MfArgs a) {
                     for (int i = 0; i < 2; i++) {
                         const int r = 16 * mb + 4 * grp + (mw == 0 ? 0 : 2) + i;
                         if (r >= tile.m) continue;
-                        const float own = (mw == 0 ? tot[mb][i] : tot[mb][2 + i]) * meta_sa[r], other = xv[r * S::RPB + wrow + l16];
+                        const float own = mw == 0 ? tot[mb][i] : tot[mb][2 + i], other = xv[r * S::RPB + wrow + l16];
                         float g = mw == 0 ? own : other, u = mw == 0 ? other : own, o;
                         if (a.act == CW_ACT_SILU) {
                             o = g / (1.0f + expf(-g)) * u;
@@ -394,7 +418,7 @@ __global__ __launch_bounds__(512, 4) void k_gms(const MfArgs a) {
                     const int r = 16 * mb + 4 * grp + i;
                     if (r >= tile.m || n >= a.n) continue;
                     float *p = a.dn + blockIdx.y * a.split_stride + (int64_t)meta_pick[r] * a.n + n;
-                    const float v = tot[mb][i] * meta_sa[r];
+                    const float v = tot[mb][i];
                     if (split) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // at the coherence point
                     else *p = v;
                 }
@@ -406,66 +430,69 @@ __global__ __launch_bounds__(512, 4) void k_gms(const MfArgs a) {
 
 // ------------------------------------------------------------------------------ pack
 
-// One wave per row, as k_pack_f16: hi and lo of every value under the row's power-of-two scale (the
-// largest value in [2^14, 2^15)), then, with SUMS, 32 halves per super-block: the 8 sub-block sums
-// over 32 as hi, as lo, and 16 zeros.
+// One wave per NV * 256 values (blockIdx.y) of a row: hi and lo (times LO) of every value under a power of two per 256
+// that brings their largest into [2^14, 2^15) (ascale: its inverse, one per 256), then, with SUMS, 32 halves
+// per super-block: the 8 sub-block sums over 32 as hi, as two terms below it (times LO; together exact) and
+// 8 zeros. 256 values that hold an infinity go in as +-2^14 for the infinities and 0 for the rest under an
+// infinite ascale: every product then has the infinity's sign, or is a NaN where the weight is 0, as in f32
+// (a NaN stays one).
 template <int NV, bool SUMS>
 __global__ __launch_bounds__(256) void k_pack_split(const float *x, int rows, int k, int ldx, uint16_t *a16, int lda, float *ascale,
                                                     PackExtra e) {
-    pack_extra(e);
-    const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (blockIdx.y == 0) pack_extra(e);
+    const int n_sb = (k + 255) / 256, row = blockIdx.x * 4 + (threadIdx.x >> 6), sb0 = NV * blockIdx.y, lane = threadIdx.x & 63;
     if (row >= rows) return;
     const float *xr = x + (int64_t)row * ldx;
     float4 v[NV];
-    float m = 0.f;
 #pragma unroll
-    for (int i = 0; i < NV; i++) v[i] = *(const float4 *)(xr + min(4 * lane + 256 * i, k - 4));
-#pragma unroll
-    for (int i = 0; i < NV; i++) {
-        if (4 * lane + 256 * i >= k) v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-        m = fmaxf(m, fmaxf(fmaxf(fabsf(v[i].x), fabsf(v[i].y)), fmaxf(fabsf(v[i].z), fabsf(v[i].w))));
-    }
-    m = wave_max(m);
-    int ex = 0;
-    if (m > 0.f && m < INFINITY) {
-        frexpf(m, &ex);
-        ex = min(15 - ex, 126);  // (a row of values below 2^-111 keeps a finite scale)
-    }
-    const float sc = ldexpf(1.0f, ex);
+    for (int i = 0; i < NV; i++) v[i] = *(const float4 *)(xr + min(4 * lane + 256 * (sb0 + i), k - 4));
     uint16_t *o = a16 + (int64_t)row * lda;
-    auto hi_lo = [](float f, uint32_t &h, uint32_t &l) {
-        const _Float16 a = (_Float16)f;
-        const float rest = f - (float)a;
-        h = __builtin_bit_cast(uint16_t, a);
-        l = __builtin_bit_cast(uint16_t, (_Float16)(fabsf((float)a) < INFINITY ? rest : 0.f));  // an infinity (or NaN) has no rest
-    };
+    auto half = [](float f) -> uint32_t { return __builtin_bit_cast(uint16_t, (_Float16)f); };
 #pragma unroll
     for (int i = 0; i < NV; i++) {
-        const int c = 4 * lane + 256 * i;
-        const float f[4] = {v[i].x * sc, v[i].y * sc, v[i].z * sc, v[i].w * sc};
+        const int sb = sb0 + i, c = 4 * lane + 256 * sb;
+        if (sb >= n_sb) break;
+        float f[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+#pragma unroll
+        for (int q = 0; q < 4; q++) f[q] = c < k ? f[q] : 0.f;
+        const float m = wave_max(fmaxf(fmaxf(fabsf(f[0]), fabsf(f[1])), fmaxf(fabsf(f[2]), fabsf(f[3]))));
+        float inv = INFINITY;
+        if (m < INFINITY) {
+            int ex = 0;
+            if (m > 0.f) {
+                frexpf(m, &ex);
+                ex = min(15 - ex, 126);  // (values below 2^-111 keep a finite scale)
+            }
+            const float sc = ldexpf(1.0f, ex);
+#pragma unroll
+            for (int q = 0; q < 4; q++) f[q] *= sc;
+            inv = ldexpf(1.0f, -ex);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; q++) f[q] = fabsf(f[q]) < INFINITY ? 0.f : f[q] == f[q] ? copysignf(16384.f, f[q]) : f[q];
+        }
+        if (lane == 0) ascale[(int64_t)row * n_sb + sb] = inv;
         if (c < k) {
             uint32_t h[4], l[4];
 #pragma unroll
-            for (int q = 0; q < 4; q++) hi_lo(f[q], h[q], l[q]);
+            for (int q = 0; q < 4; q++) {
+                h[q] = half(f[q]);
+                l[q] = half((f[q] - (float)(_Float16)f[q]) * LO);
+            }
             *(uint2 *)(o + c) = make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
             *(uint2 *)(o + k + c) = make_uint2(l[0] | l[1] << 16, l[2] | l[3] << 16);
         }
         if constexpr (SUMS) {
-            const float s = group_sum<8>((f[0] + f[1]) + (f[2] + f[3])) * (1.0f / 32);
-            uint32_t h, l;
-            hi_lo(s, h, l);
-            if (256 * i < k) {  // (whole super-blocks)
-                uint16_t *so = o + 2 * k + 32 * i;
-                if ((lane & 7) == 0) {
-                    so[lane >> 3] = (uint16_t)h;
-                    so[8 + (lane >> 3)] = (uint16_t)l;
-                } else if ((lane & 7) <= 2) {
-                    so[8 + 8 * (lane & 7) + (lane >> 3)] = 0;
-                }
-            }
+            // in f64: through the codes' centre the sums carry the part that all weights of a sub-block share
+            double s = ((double)f[0] + f[1]) + ((double)f[2] + f[3]);
+#pragma unroll
+            for (int d = 1; d < 8; d <<= 1) s += __shfl_xor(s, d);
+            s *= 1.0 / 32;
+            const float h = (float)(_Float16)(float)s, r = (float)((s - h) * LO), l = (float)(_Float16)r;
+            const uint32_t t[4] = {half(h), half(l), half((float)((s - h) * LO - l)), 0u};
+            if ((lane & 7) < 4) o[2 * k + 32 * sb + 8 * (lane & 7) + (lane >> 3)] = (uint16_t)((lane & 2) ? (lane & 1) ? t[3] : t[2] : (lane & 1) ? t[1] : t[0]);
         }
     }
-    if (lane == 0) ascale[row] = ldexpf(1.0f, -ex);
 }
 
 // ------------------------------------------------------------------------------ launchers
@@ -476,23 +503,25 @@ bool split_supported(int dtype) {
 static bool has_min(int dtype) { return dtype == CW_Q4_K || dtype == CW_Q5_K; }
 // halves of a packed row (a multiple of 8: rows start on 16 bytes)
 int split_row(int dtype, int64_t k) { return (int)(2 * k + (has_min(dtype) ? k / 256 * 32 : 0)); }
+int split_scales(int64_t k) { return (int)((k + 255) / 256); }
 
 int pack_rows_split(int dtype, const float *x, int rows, int k, int ldx, uint16_t *a16, float *ascale, hipStream_t s,
                     const PackExtra *extra) {
     if (rows == 0) return CW_OK;
     if (k % 32 || ldx % 4) return set_error(CW_ENOTSUP, "pack: row of %d (stride %d) is not whole K-steps", k, ldx);
-    const dim3 grid((rows + 3) / 4);
-    const int nv = (k + 255) / 256, lda = split_row(dtype, k);
+    if (k > 8192) return set_error(CW_ENOTSUP, "pack: rows of %d above 8192", k);
+    // two super-blocks per wave, four where the rows fill the device with those
+    const int lda = split_row(dtype, k), n_sb = split_scales(k), nv = (int64_t)rows * n_sb >= 16384 ? 4 : 2;
+    const dim3 grid((unsigned)((rows + 3) / 4), (unsigned)((n_sb + nv - 1) / nv)), block(256);
     const PackExtra e = extra ? *extra : PackExtra{};
-#define CW_PACK(N) \
-    if (nv <= N) { \
-        if (has_min(dtype)) hipLaunchKernelGGL((k_pack_split<N, true>), grid, dim3(256), 0, s, x, rows, k, ldx, a16, lda, ascale, e); \
-        else hipLaunchKernelGGL((k_pack_split<N, false>), grid, dim3(256), 0, s, x, rows, k, ldx, a16, lda, ascale, e); \
-        return check_launch("k_pack_split"); \
-    }
-    CW_PACK(2) CW_PACK(4) CW_PACK(8) CW_PACK(12) CW_PACK(16) CW_PACK(32)
+#define CW_PACK(N, S) hipLaunchKernelGGL((k_pack_split<N, S>), grid, block, 0, s, x, rows, k, ldx, a16, lda, ascale, e)
+    const bool sums = has_min(dtype);
+    if (nv == 2 && sums) CW_PACK(2, true);
+    else if (nv == 2) CW_PACK(2, false);
+    else if (sums) CW_PACK(4, true);
+    else CW_PACK(4, false);
 #undef CW_PACK
-    return set_error(CW_ENOTSUP, "pack: rows of %d above 8192", k);
+    return check_launch("k_pack_split");
 }
 
 template <class SF, int MODE>
@@ -537,7 +566,7 @@ constexpr int RPB2 = SpShape<SQ6_K, 2>::RPB, PER_CU2 = SpShape<SQ6_K, 2>::PER_CU
 size_t split_dense_workspace(int dtype, int64_t m, int64_t n, int64_t k) {
     int split_st;
     const int S = dense_splits(RPB2, 8, PER_CU2, m, n, k, split_st), tiles = (int)((m + MF_MT - 1) / MF_MT);
-    return al256((size_t)m * split_row(dtype, k) * 2) + al256(m * 4) + al256(tiles * sizeof(MfTile)) + al256(4) +
+    return al256((size_t)m * split_row(dtype, k) * 2) + al256((size_t)m * split_scales(k) * 4) + al256(tiles * sizeof(MfTile)) + al256(4) +
            (S > 1 ? al256((size_t)S * m * n * 4) + al256((size_t)gemm_items(tiles, RPB2, n) * 4) : 0);
 }
 int split_dense(int dtype, const uint8_t *w, int64_t row_bytes, int n, int k, const float *x, int m, float *y, void *ws, size_t ws_bytes,
@@ -548,7 +577,7 @@ int split_dense(int dtype, const uint8_t *w, int64_t row_bytes, int n, int k, co
     const int S = dense_splits(RPB2, 8, PER_CU2, m, n, k, split_st), tiles_n = (m + MF_MT - 1) / MF_MT;
     uint8_t *p = (uint8_t *)ws;
     uint16_t *x16 = (uint16_t *)p; p += al256((size_t)m * split_row(dtype, k) * 2);
-    float *xs = (float *)p; p += al256((size_t)m * 4);
+    float *xs = (float *)p; p += al256((size_t)m * split_scales(k) * 4);
     MfTile *tiles = (MfTile *)p; p += al256((size_t)tiles_n * sizeof(MfTile));
     int *n_tiles = (int *)p; p += al256(4);
     float *part = nullptr;

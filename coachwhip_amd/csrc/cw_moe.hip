@@ -220,9 +220,9 @@ static MoeLayout layout(const cw_moe_desc *d, int T, bool allow_split = true) {
         const bool gx = mxfp4_scaled_for(d->dtype[0], d->hidden), dx = mxfp4_scaled_for(d->dtype[2], P);
         const size_t xrow = L.split ? split_row(d->dtype[0], d->hidden) : d->hidden, hrow = L.split ? split_row(d->dtype[2], P) : P;
         L.x16 = off; off = align256(off + (gx ? fp6_rows_bytes(T, d->hidden) : (size_t)T * xrow * 2));
-        L.xscale = off; off = align256(off + (size_t)T * 4);
+        L.xscale = off; off = align256(off + (size_t)T * (L.split ? split_scales(d->hidden) : 1) * 4);
         L.h16 = off; off = align256(off + (dx ? fp6_rows_bytes((int64_t)TK, P) : TK * hrow * 2));
-        L.hscale = off; off = align256(off + TK * 4);
+        L.hscale = off; off = align256(off + TK * (L.split ? split_scales(P) : 1) * 4);
         L.dn = off; off = align256(off + TK * (size_t)d->hidden * 4);
     }
     L.total = off;

@@ -103,8 +103,9 @@ int cw_dequantize(int dtype, const void *blocks, int64_t n_elems, float *out, cw
  * From 2 rows of x (Q4_K) or 8 rows (the other formats) the product runs as an MFMA GEMM on
  * fp16-rounded activations (rel-L2 about 3e-4 against f64) and needs the workspace; below that
  * it is one f32 matvec per row. Q5_K and Q6_K keep f32 accuracy at every m: a matvec per row, or, for
- * as many rows as pay for it, a GEMM on the activations as two fp16 terms (it needs the workspace; a
- * call without one takes the matvecs). ws may be NULL when cw_qmatmul_workspace_size returns 0. */
+ * as many rows as pay for it, a GEMM on the activations as two fp16 terms, which hold a value to 2^-23
+ * of itself, or to 2^-52 of the largest of its 256-weight block where that is more (it needs the
+ * workspace; a call without one takes the matvecs). ws may be NULL when cw_qmatmul_workspace_size returns 0. */
 size_t cw_qmatmul_workspace_size(int dtype, int64_t n, int64_t k, int64_t m);
 int cw_qmatmul(int dtype, const void *w, int64_t n, int64_t k, const float *x, int64_t m,
                float *y, void *ws, size_t ws_bytes, cw_stream_t stream);

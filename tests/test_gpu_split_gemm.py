@@ -113,7 +113,7 @@ def _call(layer, x, logits, entry="workspace", ws_bytes=None):
 
 # no override: every token picks all four experts, 264 million weights beyond the distinct ones at 15 tokens
 # and 246 million at 14 of the second shape
-@pytest.mark.parametrize("pair", [(F.Q4_K, F.Q4_K), (F.Q8_0, F.Q8_0), (F.Q4_K, F.Q8_0), (F.Q4_K, F.Q6_K)],
+@pytest.mark.parametrize("pair", [(F.Q4_K, F.Q4_K), (F.Q8_0, F.Q8_0), (F.Q4_K, F.Q8_0), (F.Q8_0, F.Q4_K), (F.Q4_K, F.Q6_K)],
                          ids=lambda p: F.NAMES[p[0]] + "-" + F.NAMES[p[1]])
 @pytest.mark.parametrize("tokens,hidden,inter", [(15, 1024, 1536), (14, 2048, 768)])
 def test_layer_by_the_rule_and_with_less_workspace(pair, tokens, hidden, inter, monkeypatch):
@@ -173,3 +173,109 @@ def test_dense_by_the_rule_and_without_workspace(dtype, monkeypatch):
     plain = ops.QMatMul(ops.QTensor.from_blocks(raw, dtype, (n, k))).forward(xd).cpu().numpy()
     assert np.array_equal(got["short"], plain) and np.array_equal(got["none"], plain) and not np.array_equal(got["gemm"], plain)
     assert O.rel_l2(got["gemm"], want) <= min(REL_L2, 2 * O.rel_l2(plain, want))
+
+
+def _outlier_blocks(dtype, n, k, rng):
+    """Weights that are 0 where the test puts large activations: super-block 0 (its scale), and column 300 (Q6_K:
+    the code 32) or the sub-block around it (Q5_K: its scale and minimum)."""
+    raw = synth.random_blocks(dtype, n * k, rng).reshape(n, k // 256, -1).copy()
+    o = F.D_OFFSET[dtype]
+    raw[:, 0, o:o + (4 if dtype == F.Q5_K else 2)] = 0
+    if dtype == F.Q5_K:  # sub-block 1: the low 6 bits of scale bytes 1 and 5
+        raw[:, 1, 5] &= 0xC0
+        raw[:, 1, 9] &= 0xC0
+    else:  # quadrant 1, weight 12: the low nibble of ql[44], bits 2 and 3 of qh[12]
+        raw[:, 1, 44] &= 0xF0
+        raw[:, 1, 128 + 12] = raw[:, 1, 128 + 12] & 0xF3 | 2 << 2
+    return raw.reshape(-1)
+
+
+@pytest.mark.parametrize("dtype", [F.Q5_K, F.Q6_K])
+def test_dense_outliers_against_zero_weights(dtype, monkeypatch):
+    """Large activations whose weights are 0 do not cost the others their bits: each output row is held to the f32
+    bar by itself, as the matvec's is."""
+    rng = np.random.default_rng(dtype)
+    n, k, m = 80, 1024, 24
+    raw = _outlier_blocks(dtype, n, k, rng)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[0, 7] = 2.0 ** 25
+    x[1, 200] = -(2.0 ** 60)
+    x[2, :256] *= np.float32(1e30)
+    x[3, 300] = 2.0 ** 25
+    x[4, 300] = -1e7
+    x[5, 512:] *= np.float32(1e-20)     # super-blocks of their own size
+    x[5, 300] = 3e4
+    want = O.qmatmul_f64(dtype, raw, n, k, x)
+    got, plain = (_matmul(raw, dtype, n, k, x, monkeypatch, r) for r in (1, 1000000))
+    for t in range(m):
+        err, ref = O.rel_l2(got[t], want[t]), O.rel_l2(plain[t], want[t])
+        assert err <= max(2 * ref, REL_L2), (t, err, ref)
+
+
+@pytest.mark.parametrize("dtype", [F.Q5_K, F.Q6_K])
+def test_dense_infinities_and_nans(dtype, monkeypatch):
+    """An infinite activation gives the infinity of its weight's sign, or a NaN where the weight is 0; a NaN stays one;
+    other rows do not see them."""
+    rng = np.random.default_rng(dtype + 1)
+    n, k, m = 160, 1024, 20
+    raw = _outlier_blocks(dtype, n, k, rng)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[3, 700], x[4, 300], x[5, 9], x[6, 1023], x[7, 400] = np.inf, np.inf, -np.inf, -np.inf, np.nan
+    x[8, 600], x[8, 601], x[9, 600], x[9, 900] = np.inf, np.nan, np.inf, -np.inf
+    with np.errstate(invalid="ignore"):
+        want = O.qmatmul_f64(dtype, raw, n, k, x)
+    got = _matmul(raw, dtype, n, k, x, monkeypatch, 1)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.isnan(want[7]).all() and np.isnan(want[4]).all()
+    inf = np.isinf(want)
+    assert inf[3].any() and inf[6].any() and np.array_equal(got[inf], want[inf].astype(np.float32))
+    live = np.isfinite(want).all(1)
+    assert live.sum() == m - 7 and O.rel_l2(got[live], want[live]) <= REL_L2
+
+
+# rows of Q8_0 that end inside a stage, beside whole super-blocks of the other format
+@pytest.mark.parametrize("pair,tokens,hidden,inter", [((F.Q8_0, F.Q6_K), 33, 544, 256), ((F.Q6_K, F.Q8_0), 90, 512, 288), ((F.Q8_0, F.Q5_K), 20, 32, 512)],
+                         ids=str)
+def test_layer_of_ragged_rows(pair, tokens, hidden, inter, monkeypatch):
+    monkeypatch.setenv("CWMOE_PREFILL_MIN_TOKENS", "16")
+    rng = np.random.default_rng(hidden)
+    w = synth.moe_weights(6, 3, hidden, inter, (pair[0],) + pair, rng)
+    layer = ops.MoeLayer(*_banks(w, 6), n_experts=6, top_k=3)
+    x, logits = rng.standard_normal((tokens, hidden)).astype(np.float32), rng.standard_normal((tokens, 6)).astype(np.float32)
+    want = O.moe_layer(w, x, logits)[0]
+    assert O.rel_l2(_call(layer, ops.to_device(x), ops.to_device(logits)), want) <= 2 * REL_L2
+
+
+@pytest.mark.parametrize("pair", [(F.Q4_K, F.Q6_K), (F.Q5_K, F.Q8_0), (F.Q6_K, F.Q5_K)], ids=lambda p: F.NAMES[p[0]] + "-" + F.NAMES[p[1]])
+def test_layer_with_biases_padding_and_slots(pair, monkeypatch):
+    """The clamped SwiGLU with biases per expert, hidden rows padded with zeros, a permuted slot table, and a
+    slot past the bank (NaN rows)."""
+    monkeypatch.setenv("CWMOE_PREFILL_MIN_TOKENS", "16")
+    rng = np.random.default_rng(pair[0])
+    experts, slots, top_k, hidden, inter, pad, tokens = 24, 12, 4, 512, 512, 768, 61
+    w = synth.moe_weights(experts, top_k, hidden, inter, (pair[0],) + pair, rng, n_slots=slots, act=1, pad=pad)
+    w.bias = [20 * b for b in w.bias]
+    shapes = [(inter, hidden)] * 2 + [(hidden, pad)]
+    banks = [ops.ExpertBank.from_blocks(w.host[m], w.dtypes[m], *s, slots) for m, s in enumerate(shapes)]
+    table = np.full(experts, 0xFFFFFFFF, np.uint32)
+    resident = rng.choice(experts, slots, replace=False)
+    table[resident] = rng.permutation(slots)
+    # (x small: the clamp leaves most of the gates and ups to their weights)
+    x = (rng.standard_normal((tokens, hidden)) * 2.0 ** -8).astype(np.float32)
+    logits = rng.standard_normal((tokens, experts)).astype(np.float32)
+    logits[:, table == 0xFFFFFFFF] -= np.float32(1e30)
+    want, wids, _, _ = O.moe_layer(w, x, logits, slot_table=table, n_slots=slots)
+    act = ops.ExpertAct.clamped_swiglu(w.alpha, w.limit, *[ops.to_device(b) for b in w.bias], pad=pad)
+    xd, ld = ops.to_device(x), ops.to_device(logits)
+
+    def run(tab):
+        layer = ops.MoeLayer(*banks, n_experts=experts, top_k=top_k, act=act, slot_table=ops.to_device(tab))
+        out, ids, _ = layer.forward(xd, ld)
+        assert np.array_equal(ids.cpu().numpy().view(np.uint32), wids)
+        return out.cpu().numpy()
+
+    assert O.rel_l2(run(table), want) <= 2 * REL_L2
+    bad = wids[0, 0]
+    table[bad] = slots
+    out = run(table)
+    hit = (wids == bad).any(1)
+    assert np.isnan(out[hit]).all() and O.rel_l2(out[~hit], want[~hit]) <= 2 * REL_L2
