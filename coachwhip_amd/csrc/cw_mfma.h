@@ -9,9 +9,9 @@ constexpr int MF_MB = 5;            // MFMA blocks of 16 picks per tile
 constexpr int MF_MT = 16 * MF_MB;   // picks per tile: 80 keeps the piles of a 1,500-token batch over
                                     // 256 experts (about 47 picks each) at one tile per expert
 
-// A tile: m picks of one slot's pile from pile position pos0, and the expert they were routed to
-// (every pick of a pile reads one slot, so one expert; the slot itself when the piles were built
-// without the picks' expert ids).
+// A tile: m picks of one slot's pile from pile position pos0, and an expert they were routed to (the slot
+// itself when the piles were built without the picks' expert ids). Every pick of a pile reads one slot; all
+// of a pile by experts were routed to the tile's expert.
 struct MfTile {
     int slot, pos0, m, expert;
 };
@@ -90,10 +90,10 @@ enum { K_NATURAL = 0, K_PAIRS = 1, K_OCTETS = 2 };
 inline int k_order(int dtype) {
     return dtype == CW_MXFP4 ? K_PAIRS : dtype == CW_Q8_0 || dtype == CW_IQ4_XS ? K_NATURAL : K_OCTETS;
 }
-// one block: expert piles of the (slot) picks, and the tile list
-int mfma_piles(const uint32_t *slots, const uint32_t *ids, int TK, int K, int n_slots, int *pile_pick, int *pile_tok, MfTile *tiles,
-               int *n_tiles, hipStream_t s);
-int max_tiles(int TK, int n_slots);
+// one block: piles of the picks by slot, or by expert where n_experts is not 0, and the tile list
+int mfma_piles(const uint32_t *slots, const uint32_t *ids, int TK, int K, int n_slots, int n_experts, int *pile_pick, int *pile_tok,
+               MfTile *tiles, int *n_tiles, hipStream_t s);
+int max_tiles(int TK, int n_piles);
 // rows x k f32 -> fp16 rows (ld = k, K order as given) with per-row power-of-two scales
 int pack_rows_f16(const float *x, int rows, int k, int ldx, uint16_t *a16, float *ascale, hipStream_t s,
                   const PackExtra *extra = nullptr, int order = K_NATURAL);

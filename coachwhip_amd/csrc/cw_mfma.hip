@@ -548,14 +548,18 @@ __device__ __forceinline__ int wave_incl_scan(int v, int lane) {
     return v;
 }
 
-// One block: histogram of slots, exclusive scans, scatter of picks into per-slot piles, tiles.
+// One block: histogram of slots (or experts), exclusive scans, scatter of picks into their piles, tiles.
 // Each thread reads its (up to) PILE_PER slots into registers before using any, so the loads
 // overlap, and keeps them for the scatter; the order of picks inside a pile does not matter
 // (every pick's outputs are computed independently of the other rows of its tile). Up to
 // PILE_LDS picks, the scatter goes to LDS and the piles leave in coalesced stores (random 4-byte
 // stores from one CU cost a memory transaction each).
+// BY_EXPERT: a pile per expert (n_keys of them) instead of per slot: with a bias per expert, picks that
+// share a slot but not an expert (experts that the bank does not hold all read slot 0) need tiles of their
+// own.
 constexpr int PILE_PER = 16, PILE_LDS = 12288;
-__global__ __launch_bounds__(1024) void k_piles(const uint32_t *slots, const uint32_t *ids, int TK, int K, int n_slots,
+template <bool BY_EXPERT>
+__global__ __launch_bounds__(1024) void k_piles(const uint32_t *slots, const uint32_t *ids, int TK, int K, int n_slots, int n_keys,
                                                  int *pile_pick, int *pile_tok, MfTile *tiles, int *n_tiles) {
     __shared__ int cnt[1024], off[1024], cur[1024], rep[1024], wtot[16], wttot[16], wftot[16];
     __shared__ int staged[PILE_LDS];
@@ -565,23 +569,23 @@ __global__ __launch_bounds__(1024) void k_piles(const uint32_t *slots, const uin
     rep[tid] = 0;
     const bool one = TK <= 1024 * PILE_PER;  // the common case: every slot read once, kept in registers
     uint32_t v[PILE_PER];
+    // the pile of pick i (none past the last one, or for a slot past the bank)
+    auto key = [&](int i) __attribute__((always_inline)) -> uint32_t {
+        if (i >= TK) return 0xFFFFFFFFu;
+        if constexpr (BY_EXPERT) return slots[i] < (uint32_t)n_slots ? ids[i] : 0xFFFFFFFFu;
+        else return slots[i];
+    };
 #pragma unroll
-    for (int q = 0; q < PILE_PER; q++) {
-        const int i = q * 1024 + tid;
-        v[q] = i < TK ? slots[i] : 0xFFFFFFFFu;
-    }
+    for (int q = 0; q < PILE_PER; q++) v[q] = key(q * 1024 + tid);
     __syncthreads();
     for (int c0 = 0; c0 < TK; c0 += 1024 * PILE_PER) {
         if (c0) {
 #pragma unroll
-            for (int q = 0; q < PILE_PER; q++) {
-                const int i = c0 + q * 1024 + tid;
-                v[q] = i < TK ? slots[i] : 0xFFFFFFFFu;
-            }
+            for (int q = 0; q < PILE_PER; q++) v[q] = key(c0 + q * 1024 + tid);
         }
 #pragma unroll
         for (int q = 0; q < PILE_PER; q++)
-            if (v[q] < (uint32_t)n_slots) {
+            if (v[q] < (uint32_t)n_keys) {
                 atomicAdd(&cnt[v[q]], 1);
                 atomicMax(&rep[v[q]], c0 + q * 1024 + tid);  // a pick of the slot, for its expert id
             }
@@ -591,7 +595,7 @@ __global__ __launch_bounds__(1024) void k_piles(const uint32_t *slots, const uin
     // 16 wave totals. The tile list holds every slot's first tile, then the later tiles of the
     // slots with more than MF_MT picks: the GEMMs hand out work items in list order, so the last
     // round of items, which only some blocks run, takes the (smaller) remainder tiles.
-    const int c = tid < n_slots ? cnt[tid] : 0;
+    const int c = tid < n_keys ? cnt[tid] : 0;
     const int tc = (c + MF_MT - 1) / MF_MT, fc = c > 0 ? 1 : 0;
     const int ic = wave_incl_scan(c, lane), itc = wave_incl_scan(tc, lane), ifc = wave_incl_scan(fc, lane);
     if (lane == 63) {
@@ -612,24 +616,21 @@ __global__ __launch_bounds__(1024) void k_piles(const uint32_t *slots, const uin
     const int my_off = wc + ic - c, my_toff = wtc + itc - tc, my_f = wfc + ifc - fc;
     if (tid == 1023) *n_tiles = my_toff + tc;
     off[tid] = my_off;
-    if (tid < n_slots) {
-        const int ex = ids && c > 0 ? (int)ids[rep[tid]] : tid;
+    if (tid < n_keys) {
+        const int ex = !BY_EXPERT && ids && c > 0 ? (int)ids[rep[tid]] : tid, sl = BY_EXPERT && c > 0 ? (int)slots[rep[tid]] : tid;
         for (int q = 0; q < tc; q++)
-            tiles[q == 0 ? my_f : nf + (my_toff - my_f) + q - 1] = MfTile{tid, my_off + q * MF_MT, min(MF_MT, c - q * MF_MT), ex};
+            tiles[q == 0 ? my_f : nf + (my_toff - my_f) + q - 1] = MfTile{sl, my_off + q * MF_MT, min(MF_MT, c - q * MF_MT), ex};
     }
     __syncthreads();
     for (int c0 = 0; c0 < TK; c0 += 1024 * PILE_PER) {
         if (!one) {
 #pragma unroll
-            for (int q = 0; q < PILE_PER; q++) {
-                const int i = c0 + q * 1024 + tid;
-                v[q] = i < TK ? slots[i] : 0xFFFFFFFFu;
-            }
+            for (int q = 0; q < PILE_PER; q++) v[q] = key(c0 + q * 1024 + tid);
         }
 #pragma unroll
         for (int q = 0; q < PILE_PER; q++) {
             const int i = c0 + q * 1024 + tid;
-            if (v[q] < (uint32_t)n_slots) {
+            if (v[q] < (uint32_t)n_keys) {
                 const int pos = off[v[q]] + atomicAdd(&cur[v[q]], 1);
                 if (TK <= PILE_LDS) {
                     staged[pos] = i;
@@ -759,12 +760,13 @@ bool mfma_supported(int dtype) {
            dtype == CW_Q2_K || dtype == CW_IQ3_XXS || dtype == CW_IQ4_XS || dtype == CW_MXFP4_R16;
 }
 
-int max_tiles(int TK, int n_slots) { return (TK + MF_MT - 1) / MF_MT + (n_slots < TK ? n_slots : TK); }
+int max_tiles(int TK, int n_piles) { return (TK + MF_MT - 1) / MF_MT + (n_piles < TK ? n_piles : TK); }
 
-int mfma_piles(const uint32_t *slots, const uint32_t *ids, int TK, int K, int n_slots, int *pile_pick, int *pile_tok, MfTile *tiles,
-               int *n_tiles, hipStream_t s) {
-    if (n_slots > 1024) return set_error(CW_ENOTSUP, "mfma: %d slots (1024 max)", n_slots);
-    hipLaunchKernelGGL(k_piles, dim3(1), dim3(1024), 0, s, slots, ids, TK, K, n_slots, pile_pick, pile_tok, tiles, n_tiles);
+int mfma_piles(const uint32_t *slots, const uint32_t *ids, int TK, int K, int n_slots, int n_experts, int *pile_pick, int *pile_tok,
+               MfTile *tiles, int *n_tiles, hipStream_t s) {
+    if (n_slots > 1024 || n_experts > 1024) return set_error(CW_ENOTSUP, "mfma: %d slots, %d experts (1024 max)", n_slots, n_experts);
+    if (n_experts) hipLaunchKernelGGL(k_piles<true>, dim3(1), dim3(1024), 0, s, slots, ids, TK, K, n_slots, n_experts, pile_pick, pile_tok, tiles, n_tiles);
+    else hipLaunchKernelGGL(k_piles<false>, dim3(1), dim3(1024), 0, s, slots, ids, TK, K, n_slots, n_slots, pile_pick, pile_tok, tiles, n_tiles);
     return check_launch("k_piles");
 }
 

@@ -192,6 +192,11 @@ static int check_desc(const cw_moe_desc *d, int T) {
     return CW_OK;
 }
 
+// Gate/up biases are per expert and a slot table may send several experts to one slot (those that the bank
+// does not hold read slot 0): the GEMMs' piles then go by expert, whose tiles know their bias rows
+static bool piles_by_expert(const cw_moe_desc *d) { return d->slot_table && (d->bias[0] || d->bias[1]); }
+static int n_piles(const cw_moe_desc *d) { return d->slot_table && !piles_by_expert(d) ? d->n_slots : d->n_experts; }
+
 // allow_split: off for callers whose scratch holds the matvecs' layout but not the split GEMMs'
 static MoeLayout layout(const cw_moe_desc *d, int T, bool allow_split = true) {
     const size_t TK = (size_t)T * d->top_k;
@@ -211,10 +216,9 @@ static MoeLayout layout(const cw_moe_desc *d, int T, bool allow_split = true) {
     L.split = allow_split && split_path(d, T);
     L.grouped = L.split || grouped_path(d, T);
     if (L.grouped) {
-        const int n_slots = d->slot_table ? d->n_slots : d->n_experts;
         L.pile_pick = off; off = align256(off + TK * 4);
         L.pile_tok = off; off = align256(off + TK * 4);
-        L.tiles = off; off = align256(off + (size_t)max_tiles((int)TK, n_slots) * sizeof(MfTile));
+        L.tiles = off; off = align256(off + (size_t)max_tiles((int)TK, n_piles(d)) * sizeof(MfTile));
         L.n_tiles = off; off = align256(off + 4);
         // fp16 rows, or for MXFP4 on the scaled MFMA the rows packed as FP6 terms
         const bool gx = mxfp4_scaled_for(d->dtype[0], d->hidden), dx = mxfp4_scaled_for(d->dtype[2], P);
@@ -242,7 +246,7 @@ static int moe_grouped(const cw_moe_desc *d, const MoeArgs &a, const MoeLayout &
     }
     int *pile_pick = (int *)(base + L.pile_pick), *pile_tok = (int *)(base + L.pile_tok), *n_tiles = (int *)(base + L.n_tiles);
     MfTile *tiles = (MfTile *)(base + L.tiles);
-    if ((rc = mfma_piles(slots, a.ids, TK, K, a.n_slots, pile_pick, pile_tok, tiles, n_tiles, s))) return rc;
+    if ((rc = mfma_piles(slots, a.ids, TK, K, a.n_slots, piles_by_expert(d) ? a.E : 0, pile_pick, pile_tok, tiles, n_tiles, s))) return rc;
     uint16_t *x16 = (uint16_t *)(base + L.x16), *h16 = (uint16_t *)(base + L.h16);
     float *xscale = (float *)(base + L.xscale), *hscale = (float *)(base + L.hscale);
     // MXFP4 matrices run on the block-scaled MFMA (activations as FP6 terms), the others on fp16 MFMA
@@ -254,7 +258,7 @@ static int moe_grouped(const cw_moe_desc *d, const MoeArgs &a, const MoeLayout &
     // gate/up and down both on the scaled MFMA: gate/up packs the hidden rows itself
     const bool fuse_h = gx && dx;
     if (!fuse_h && P > a.I && (rc = fill_zero(a.h, (int64_t)TK * P, s))) return rc;
-    const int tmax = max_tiles(TK, a.n_slots);
+    const int tmax = max_tiles(TK, n_piles(d));
 
     MfArgs g = {};
     g.w0 = a.wg;
@@ -596,7 +600,7 @@ int cw_matmul_id_grouped(int dtype, int64_t n, int64_t k, int64_t n_slots, int64
     MfTile *tiles = (MfTile *)(base + L.tiles);
     uint16_t *x16 = (uint16_t *)(base + L.x16);
     float *xscale = (float *)(base + L.xscale);
-    if ((rc = mfma_piles(ids, nullptr, TK, K, (int)n_slots, pile_pick, pile_tok, tiles, n_tiles, s))) return rc;
+    if ((rc = mfma_piles(ids, nullptr, TK, K, (int)n_slots, 0, pile_pick, pile_tok, tiles, n_tiles, s))) return rc;
     const bool gx = mxfp4_scaled_for(dtype, k);
     if (gx) rc = pack_rows_fp6(x, xpp ? TK : T, (int)k, (int)k, (uint8_t *)x16, s);
     else rc = pack_rows_f16(x, xpp ? TK : T, (int)k, (int)k, x16, xscale, s, nullptr, k_order(dtype));
