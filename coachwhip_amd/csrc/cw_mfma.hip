@@ -654,7 +654,7 @@ __global__ __launch_bounds__(1024) void k_piles(const uint32_t *slots, const uin
 
 // One wave per row, the row held in registers (NV float4 per lane, k <= 256*NV): scale =
 // 2^(15 - e) with max|x| in [2^(e-1), 2^e) keeps the row's largest value in [2^14, 2^15) of
-// fp16; ascale receives 1/scale.
+// fp16 (below it for rows under 2^-111); ascale receives 1/scale.
 template <int NV, int ORDER>
 __global__ __launch_bounds__(256) void k_pack_f16(const float *x, int rows, int k, int ldx, uint16_t *a16, float *ascale,
                                                   PackExtra e) {
@@ -687,7 +687,10 @@ __global__ __launch_bounds__(256) void k_pack_f16(const float *x, int rows, int 
     }
     m = wave_max(m);
     int ex = 0;
-    if (m > 0.f && m < INFINITY) { frexpf(m, &ex); ex = 15 - ex; }
+    if (m > 0.f && m < INFINITY) {
+        frexpf(m, &ex);
+        ex = min(15 - ex, 126);  // (a row of values below 2^-111 keeps a finite scale, and 1 / scale stays normal)
+    }
     const float sc = ldexpf(1.0f, ex);
     uint16_t *o = a16 + (int64_t)row * k;
     // K_OCTETS: the lane's 4 values are half (lane & 1) of octet l = (lane >> 1) & 3 of sub-block 4j + g =
