@@ -108,10 +108,16 @@ static bool qmatmul_split(int dtype, int64_t n, int64_t k, int64_t m) {
     return m > 2 && (5 * m - 12) * n * k >= 215000000ll;
 }
 
-size_t cw_qmatmul_workspace_size(int dtype, int64_t n, int64_t k, int64_t m) {
+}  // extern "C"
+size_t cw::qmatmul_required_workspace(int dtype, int64_t n, int64_t k, int64_t m) {
     if (!is_weight_type(dtype) || k <= 0 || m <= 0) return 0;
-    if (qmatmul_split(dtype, n, k, m)) return n > 0 ? cw::split_dense_workspace(dtype, m, n, k) : 0;
     return qmatmul_mfma(dtype, k, m) ? cw::mfma_dense_workspace(dtype, m, n, k) : 0;
+}
+extern "C" {
+
+size_t cw_qmatmul_workspace_size(int dtype, int64_t n, int64_t k, int64_t m) {
+    if (is_weight_type(dtype) && m > 0 && qmatmul_split(dtype, n, k, m)) return cw::split_dense_workspace(dtype, m, n, k);
+    return cw::qmatmul_required_workspace(dtype, n, k, m);
 }
 
 int cw_qmatmul(int dtype, const void *w, int64_t n, int64_t k, const float *x, int64_t m, float *y, void *ws,

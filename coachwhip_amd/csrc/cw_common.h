@@ -30,6 +30,9 @@ __host__ __device__ __forceinline__ int64_t rows16_offset(int64_t r, int b, int 
 
 // formats of expert matrices: the GGUF ones, and MXFP4 in row groups of 16
 inline bool is_expert_type(int dtype) { return is_weight_type(dtype) || dtype == CW_MXFP4_R16; }
+// workspace that cw_qmatmul cannot do without (cw_qmatmul_workspace_size adds that of the f32-accurate GEMMs,
+// which have the matvecs to fall back on)
+size_t qmatmul_required_workspace(int dtype, int64_t n, int64_t k, int64_t m);
 // bytes of a matrix of n rows: row groups of 16 hold whole groups
 inline int64_t matrix_bytes(int dtype, int64_t n, int64_t row_bytes) {
     return (dtype == CW_MXFP4_R16 ? (n + 15) / 16 * 16 : n) * row_bytes;

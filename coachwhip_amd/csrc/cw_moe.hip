@@ -519,21 +519,26 @@ __global__ void k_gate_scale_add(const float *y, const float *glog, int T, int H
 static size_t al256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 // workspace of the shared expert: gate and up rows (the hidden rows overwrite gate), down rows,
-// gate logits, and one region the three matmuls take in turn
+// gate logits, and one region the three matmuls take in turn: required, what they cannot do without; total,
+// with the f32-accurate GEMMs' (whose size does not grow with every T)
 struct SharedLayout {
-    size_t g, u, y, glog, mm, total;
+    size_t g, u, y, glog, mm, required, total;
 };
 static SharedLayout shared_layout(const cw_shared_desc *d, int T) {
     SharedLayout L;
     const size_t ti = (size_t)T * d->inter * 4, th = (size_t)T * d->hidden * 4;
-    size_t mm = cw_qmatmul_workspace_size(d->dtype[0], d->inter, d->hidden, T);
-    mm = std::max(mm, cw_qmatmul_workspace_size(d->dtype[1], d->inter, d->hidden, T));
-    mm = std::max(mm, cw_qmatmul_workspace_size(d->dtype[2], d->hidden, d->inter, T));
+    size_t mm = 0, need = 0;
+    for (int m = 0; m < 3; m++) {
+        const int64_t n = m == 2 ? d->hidden : d->inter, k = m == 2 ? d->inter : d->hidden;
+        mm = std::max(mm, cw_qmatmul_workspace_size(d->dtype[m], n, k, T));
+        need = std::max(need, qmatmul_required_workspace(d->dtype[m], n, k, T));
+    }
     L.g = 0;
     L.u = L.g + al256(ti);
     L.y = L.u + al256(ti);
     L.glog = L.y + al256(th);
     L.mm = L.glog + al256((size_t)T * 4);
+    L.required = L.mm + al256(need);
     L.total = L.mm + al256(mm);
     return L;
 }
@@ -555,13 +560,13 @@ int cw_shared_expert(const cw_shared_desc *d, const float *x, int T, float *out,
     if (T == 0) return CW_OK;
     CW_REQUIRE(x && out && d->w[0] && d->w[1] && d->w[2], "shared expert: null pointer");
     const SharedLayout L = shared_layout(d, T);
-    CW_REQUIRE(ws && ws_bytes >= L.total, "shared expert: workspace of %zu bytes, %zu needed", ws_bytes, L.total);
+    CW_REQUIRE(ws && ws_bytes >= L.required, "shared expert: workspace of %zu bytes, %zu needed", ws_bytes, L.required);
     hipStream_t s = (hipStream_t)stream;
     uint8_t *base = (uint8_t *)ws;
     float *g = (float *)(base + L.g), *u = (float *)(base + L.u), *y = (float *)(base + L.y);
     float *glog = d->gate_inp ? (float *)(base + L.glog) : nullptr;
     void *mm = base + L.mm;
-    const size_t mm_bytes = L.total - L.mm;
+    const size_t mm_bytes = std::min(ws_bytes, L.total) - L.mm;
     int rc;
     if ((rc = cw_qmatmul(d->dtype[0], d->w[0], d->inter, d->hidden, x, T, g, mm, mm_bytes, stream))) return rc;
     if ((rc = cw_qmatmul(d->dtype[1], d->w[1], d->inter, d->hidden, x, T, u, mm, mm_bytes, stream))) return rc;

@@ -282,7 +282,8 @@ typedef struct cw_shared_desc {
 /* out[t] = sigmoid(x[t] . gate_inp) * down(silu(gate x[t]) * (up x[t])), added to out when
  * accumulate != 0 (the block sums routed and shared outputs). Replaces SharedExpert::forward
  * (crates/engine/src/model_next.rs:723-742; the sum at 1430-1437). x is T rows of hidden,
- * 16-byte aligned; ws from cw_shared_expert_workspace_size. */
+ * 16-byte aligned; ws from cw_shared_expert_workspace_size. Q5_K and Q6_K matrices run without their
+ * part of it (cw_qmatmul's), as matvecs, where the workspace is smaller. */
 size_t cw_shared_expert_workspace_size(const cw_shared_desc *desc, int T);
 int cw_shared_expert(const cw_shared_desc *desc, const float *x, int T, float *out, int accumulate,
                      void *ws, size_t ws_bytes, cw_stream_t stream);
