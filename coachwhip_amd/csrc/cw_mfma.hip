@@ -159,16 +159,17 @@ __global__ __launch_bounds__(1024, 4) void k_gmm(const MfArgs a) {
             else meta_pick[tid] = mpos;
         }
 
-        // Row r of the block is row nblk*RPB + r % RPB of matrix r / RPB (rows past n read row 0).
-        // Addresses are the block's matrix base (uniform) plus 32-bit offsets (a matrix is under
-        // 4 GiB: checked at launch), so they need no 64-bit registers per row.
-        const uint8_t *wb0 = a.w0 + (int64_t)tile.slot * a.s0;
-        const uint8_t *wb1 = S::NM > 1 ? a.w1 + (int64_t)tile.slot * a.s1 : wb0;
+        // Row r of the block is row nblk*RPB + r % RPB of matrix r / RPB (rows past n read the block's
+        // first). Addresses are the first row of the block in its matrix (uniform) plus 32-bit offsets,
+        // so they need no 64-bit registers per row.
+        const int64_t row0 = (int64_t)nblk * S::RPB * a.row_bytes;
+        const uint8_t *wb0 = a.w0 + (int64_t)tile.slot * a.s0 + row0;
+        const uint8_t *wb1 = S::NM > 1 ? a.w1 + (int64_t)tile.slot * a.s1 + row0 : wb0;
         const int mw = S::NM > 1 ? wave / S::WPM : 0;  // this wave's matrix
         const int wrow = (wave - mw * S::WPM) * S::RPW;  // its first row within the matrix's N-block
-        auto row_off = [&](int r, int m) -> uint32_t {  // byte offset of row r within matrix m
-            const int n = nblk * S::RPB + (r - m * S::RPB);
-            return (uint32_t)(n < a.n ? n : 0) * (uint32_t)a.row_bytes;
+        auto row_off = [&](int r, int m) -> uint32_t {  // byte offset of row r from the block's first of matrix m
+            const int q = r - m * S::RPB;
+            return (uint32_t)(nblk * S::RPB + q < a.n ? q : 0) * (uint32_t)a.row_bytes;
         };
 
         const int n_ks = a.k / 32, n_st = (n_ks + KST - 1) / KST;
@@ -198,7 +199,7 @@ __global__ __launch_bounds__(1024, 4) void k_gmm(const MfArgs a) {
         // wave's pieces lie in one matrix and the matrix base stays scalar. A piece's row offset and its
         // place in the row's window are the same in every stage, so they are worked out once per tile
         // (the division by the window's piece count and the row's 32-bit multiply), from the 16-byte
-        // boundary at or below the matrix base: wp_off the row's first byte, wp_p the piece.
+        // boundary at or below the block's first row: wp_off the row's first byte, wp_p the piece.
         constexpr int NP = S::NM * S::RPB * W::PCS, NTW = (NP + S::NT - 1) / S::NT;
         static_assert(S::RPB * W::PCS % 64 == 0, "a wave's pieces lie in one matrix");
         const uint32_t b0 = (uint32_t)(uintptr_t)wb0 & 15, b1 = (uint32_t)(uintptr_t)wb1 & 15;
@@ -839,7 +840,7 @@ template <class MF, int MODE>
 static int launch(const MfArgs &a, int tiles_max, int splits, hipStream_t s) {
     using S = GmShape<MF, MODE>;
     if (a.k % MF::SBK) return set_error(CW_ENOTSUP, "mfma: k %d is not a multiple of %d", a.k, MF::SBK);
-    if ((int64_t)a.n * a.row_bytes > ((int64_t)1 << 32) - 16)  // (32-bit offsets from the 16-byte boundary below the matrix)
+    if ((int64_t)a.n * a.row_bytes >= ((int64_t)1 << 32))
         return set_error(CW_ENOTSUP, "mfma: a matrix of %d rows of %lld bytes is 4 GiB or more", a.n, (long long)a.row_bytes);
     const int R = run_of_tiles(tiles_max);
     const int64_t items = gemm_items(tiles_max, S::RPB, a.n);
