@@ -51,20 +51,28 @@ struct GmShape {
     // where three stages of windows fit beside it, else 2.
     static constexpr int a_bytes(int ka) { return 2 * ka * MF_MB * 64 * 16; }
     static constexpr int room(int ka) { return LDS_MAX / PER_CU - ((MF::LDS + 15) & ~15) - a_bytes(ka) - META_BYTES; }
-    static constexpr int KA = room(4) >= 3 * W_BYTES ? 4 : 2, HPS = MF::KST / KA;
+    static constexpr int KA = room(4) >= 3 * W_BYTES ? 4 : 2;
     static constexpr int NWB = room(KA) >= 3 * W_BYTES ? 3 : 2;
-    static constexpr int A_BYTES = a_bytes(KA);
+    // MXFP4, whose K-steps are the shortest (a conversion per byte, no tables), feels the barrier per part
+    // most: its ring takes what LDS the windows leave (less the kernel's static word, to whole KB), and tiles
+    // of so few pick blocks that two parts of four K-steps fit (four, 64 rows) go in those. Dense 4096 x
+    // 4096 at 16 rows 17.2 -> 16.5 us, 64 rows 25.5 -> 24.8, 80 rows (three parts of two) 28.6 -> 28.2, 8192 x
+    // 1024 at 12 rows 12.1 -> 11.8; parts of eight at 32 rows and fewer measured the same.
+    static constexpr bool WIDE = std::is_same<MF, MMXFP4>::value && KA == 2;
+    static constexpr int A_BYTES = WIDE ? (room(0) - NWB * W_BYTES - 16) / 1024 * 1024 : a_bytes(KA);
+    static constexpr int ka(int mbs) { return WIDE && 2 * 4 * mbs * 1024 <= A_BYTES ? 4 : KA; }
+    static constexpr int hps(int mbs) { return MF::KST / ka(mbs); }
     // parts of the activation ring for MBS pick blocks: a part is requested NA - 1 parts ahead, and never
     // before the windows of its stage
     static constexpr int na(int mbs) {
-        const int n = 2 * MF_MB / mbs, m = 1 + (NWB - 1) * HPS;
+        const int n = A_BYTES / (ka(mbs) * mbs * 1024), m = 1 + (NWB - 1) * hps(mbs);
         return n < m ? (n < 5 ? n : 5) : (m < 5 ? m : 5);
     }
     // Loads that may still be in flight when part hp of a stage starts: what its wave has requested after
     // the part's activations and, for the stage's first part, after the stage's windows (loads return in
-    // order). ntw: a wave's window loads per stage; ka: its activation loads per part (0 for the waves
-    // that load none).
-    static constexpr int in_flight(int hp, int NA, int ntw, int ka) {
+    // order). HPS: parts per stage; ntw: a wave's window loads per stage; ka: its activation loads per part
+    // (0 for the waves that load none).
+    static constexpr int in_flight(int hp, int HPS, int NA, int ntw, int ka) {
         int n = ka * (NA - 2);
         for (int i = 1; i <= NA - 1; i++) n += (hp - i) % HPS == 0 ? ntw : 0;  // stage starts among the parts since
         if (hp == 0) {
@@ -230,11 +238,11 @@ __global__ __launch_bounds__(1024, 4) void k_gmm(const MfArgs a) {
         // K-steps KA*p .. KA*p + KA-1 of the row (clamped to it where it may end in between: unused) into a
         // ring slot (an LDS address) of MBS pick blocks
         auto issue_a = [&](int p, uint32_t slot, auto mbs_c) __attribute__((always_inline)) {
-            constexpr int MBS = decltype(mbs_c)::value;
+            constexpr int MBS = decltype(mbs_c)::value, KA = S::ka(MBS);
             if (!stager) return;
 #pragma unroll
-            for (int kk = 0; kk < S::KA; kk++) {
-                const int ks = p * S::KA + kk;
+            for (int kk = 0; kk < KA; kk++) {
+                const int ks = p * KA + kk;
                 dma16(asrc + (MF::SBK == 32 ? min(ks, n_ks - 1) : ks) * 32, slot + (kk * MBS + wave) * 1024);
             }
         };
@@ -254,14 +262,14 @@ __global__ __launch_bounds__(1024, 4) void k_gmm(const MfArgs a) {
         // that the loads issued after it overwrite. Near an item's end, where fewer loads are in flight
         // than in_flight counts on, a part waits for all of them.
         auto stages = [&](auto mbs_c) __attribute__((always_inline)) {
-            constexpr int MBS = decltype(mbs_c)::value, NA = S::na(MBS), SLOT = S::KA * MBS * 1024;
-            const int p_lo = st_lo * S::HPS, p_hi = st_hi * S::HPS;
+            constexpr int MBS = decltype(mbs_c)::value, KA = S::ka(MBS), HPS = S::hps(MBS), NA = S::na(MBS), SLOT = KA * MBS * 1024;
+            const int p_lo = st_lo * HPS, p_hi = st_hi * HPS;
             // the loads before the first part, in the order that the parts before it would have issued them
 #pragma unroll
-            for (int q = 1 - NA < -(S::NWB - 1) * S::HPS ? 1 - NA : -(S::NWB - 1) * S::HPS; q < 0; q++) {
+            for (int q = 1 - NA < -(S::NWB - 1) * HPS ? 1 - NA : -(S::NWB - 1) * HPS; q < 0; q++) {
                 if (q + NA - 1 >= 0 && p_lo + q + NA - 1 < p_hi) issue_a(p_lo + q + NA - 1, as_lds + (q + NA - 1) * SLOT, mbs_c);
-                if (q % S::HPS == 0 && st_lo + q / S::HPS + S::NWB - 1 < st_hi)
-                    issue_w(st_lo + q / S::HPS + S::NWB - 1, ws_lds + (q / S::HPS + S::NWB - 1) * S::W_BYTES);
+                if (q % HPS == 0 && st_lo + q / HPS + S::NWB - 1 < st_hi)
+                    issue_w(st_lo + q / HPS + S::NWB - 1, ws_lds + (q / HPS + S::NWB - 1) * S::W_BYTES);
             }
             int aslot = 0, wslot = 0;  // ring slots of the current part and stage
             for (int st = st_lo; st < st_hi; st++) {
@@ -272,10 +280,10 @@ __global__ __launch_bounds__(1024, 4) void k_gmm(const MfArgs a) {
                 const uint8_t *Ap;
                 auto start_part = [&](auto hp_c) __attribute__((always_inline)) {
                     constexpr int hp = decltype(hp_c)::value;
-                    const int p = st * S::HPS + hp;
+                    const int p = st * HPS + hp;
                     const int last_w = (hp == 0 ? st - 1 : st) + S::NWB - 1;  // the last windows requested before this part
                     if (p + NA - 2 < p_hi && last_w < st_hi) {
-                        constexpr int na = S::in_flight(hp, NA, NTW, S::KA), nb = S::in_flight(hp, NA, NTW, 0);
+                        constexpr int na = S::in_flight(hp, HPS, NA, NTW, KA), nb = S::in_flight(hp, HPS, NA, NTW, 0);
                         if (stager) __builtin_amdgcn_s_waitcnt((na & 15) | ((na >> 4) << 14) | (7 << 4) | (15 << 8));
                         else __builtin_amdgcn_s_waitcnt((nb & 15) | ((nb >> 4) << 14) | (7 << 4) | (15 << 8));
                     } else {
@@ -369,7 +377,7 @@ __global__ __launch_bounds__(1024, 4) void k_gmm(const MfArgs a) {
                 };
                 auto issue_av = [&](int kk) __attribute__((always_inline)) {
 #pragma unroll
-                    for (int mb = 0; mb < MBS; mb++) av[kk & 1][mb] = *(const f16x8 *)(Ap + (((kk % S::KA) * MBS + mb) * 64 + lane) * 16);
+                    for (int mb = 0; mb < MBS; mb++) av[kk & 1][mb] = *(const f16x8 *)(Ap + (((kk % KA) * MBS + mb) * 64 + lane) * 16);
                 };
                 issue_raw(0);
                 if (1 < nke) issue_raw(1);
@@ -380,8 +388,8 @@ __global__ __launch_bounds__(1024, 4) void k_gmm(const MfArgs a) {
                 auto step = [&](auto kk_c) __attribute__((always_inline)) {
                     constexpr int kk = decltype(kk_c)::value;
                     if (kk >= nke) return;  // uniform
-                    if constexpr (kk > 0 && kk % S::KA == 0) {
-                        start_part(Ic<kk / S::KA>{});
+                    if constexpr (kk > 0 && kk % KA == 0) {
+                        start_part(Ic<kk / KA>{});
                         if constexpr (S::PF) issue_av(kk);
                     }
                     if constexpr (!S::PF) {
@@ -417,7 +425,7 @@ __global__ __launch_bounds__(1024, 4) void k_gmm(const MfArgs a) {
                     if (kk + 2 < KST && kk + 2 < nke) issue_raw(kk + 2);  // into the buffer step kk has just used
                     if (S::PF && kk + 1 < KST && kk + 1 < nke) {
                         issue_look(kk + 1);
-                        if ((kk + 1) % S::KA != 0) issue_av(kk + 1);
+                        if ((kk + 1) % KA != 0) issue_av(kk + 1);
                     }
 #pragma unroll
                     for (int mb = 0; mb < MBS; mb++)
@@ -434,9 +442,9 @@ __global__ __launch_bounds__(1024, 4) void k_gmm(const MfArgs a) {
                 // a row's last stage may end before its later parts: their barriers all the same (they
                 // were requested, and their slots count)
                 if constexpr (MF::SBK == 32) {
-                    if constexpr (S::HPS > 1) if (nke <= S::KA) start_part(Ic<1>{});
-                    if constexpr (S::HPS > 2) if (nke <= 2 * S::KA) start_part(Ic<2>{});
-                    if constexpr (S::HPS > 3) if (nke <= 3 * S::KA) start_part(Ic<3>{});
+                    if constexpr (HPS > 1) if (nke <= KA) start_part(Ic<1>{});
+                    if constexpr (HPS > 2) if (nke <= 2 * KA) start_part(Ic<2>{});
+                    if constexpr (HPS > 3) if (nke <= 3 * KA) start_part(Ic<3>{});
                 }
                 wslot = wslot + 1 == S::NWB ? 0 : wslot + 1;
             }
