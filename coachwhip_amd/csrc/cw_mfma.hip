@@ -1087,9 +1087,9 @@ __global__ __launch_bounds__(64 * W) void k_skinny_q4k(const uint8_t *w, int64_t
 // CU at most, and at most 128 KB of x per block. us per call, packed / f32: 4096 x 4096 at 2 rows 9.2 / 7.8,
 // at 8 rows 10.3 / 9.2, 4096 x 2048 at 16 rows 8.5 / 7.5, 4096 x 1024 at 16 rows 7.3 / 5.7, 512 x 512 at 16
 // rows 6.6 / 4.8. Past it the loads of x cost as much as the launch or more: 4096 x 4096 at 16 rows 12.1 /
-// 11.8, 4096 x 3072 at 16 rows 10.8 / 11.5, 8192 x 4096 at 2 rows 12.6 / 14.3, at 16 rows 16.3 / 21.4,
+// 11.8 (equal within the runs' spread), 4096 x 3072 at 16 rows 10.8 / 11.5, 8192 x 4096 at 2 rows 12.6 / 14.3, at 16 rows 16.3 / 21.4,
 // 5120 x 2048 at 16 rows 10.5 / 11.4. (A 16-wave block, k above 4,096, would not have the registers.)
-static bool skinny_f32(int n, int waves, int m) { return n <= 16 * 256 && m * waves * SKINNY_SB * 256 <= 32768; }
+static bool skinny_f32(int n, int waves, int m) { return n <= 16 * resident_blocks(1) && m * waves * SKINNY_SB * 256 <= 32768; }
 
 // 2..16 rows of Q4_K x: k_skinny_q4k, after the pack (fp16 activations and their scales) if it takes packed rows
 static int dense_skinny_q4k(const uint8_t *w, int64_t row_bytes, int n, int k, const float *x, int m, float *y, uint16_t *x16,

@@ -14,6 +14,7 @@
 
 #include "cw_common.h"
 #include "cw_device.h"
+#include "cw_mfma.h"
 #include "cw_moe_fused.h"
 #include "cw_wave.h"
 
@@ -1078,7 +1079,7 @@ __global__ __launch_bounds__(256 * G, G == 1 ? 3 : 1) void k_moe_decode(const Mo
 // blocks (of all tokens) that keep the device's CUs busy without more block starts than needed:
 // about 16 waves per CU
 static int blocks_per_token(int waves, int T, int want) {
-    const int all = 256 * 16 / waves, per = (all + T - 1) / T;
+    const int all = (int)resident_blocks(16) / waves, per = (all + T - 1) / T;
     return want < per ? want : per;
 }
 

@@ -38,6 +38,21 @@ def test_few_tokens_match_the_oracle(pair, hidden, inter, top_k, tokens):
     assert O.rel_l2(out.cpu().numpy(), want) <= REL_L2_F32
 
 
+# 256 experts and their neighbours, 512 and theirs (a lane of the routing wave holds 4, 8 or 16 logits), the most
+@pytest.mark.parametrize("experts", [255, 256, 257, 512, 513, 1024])
+def test_few_tokens_over_many_experts(experts):
+    rng = np.random.default_rng(experts)
+    w = synth.moe_weights(experts, 8, 256, 256, (F.IQ2_XXS, F.IQ2_XXS, F.IQ2_S), rng)
+    x, logits = rng.standard_normal((5, 256)).astype(np.float32), rng.standard_normal((5, experts)).astype(np.float32)
+    logits[0] = np.round(2 * logits[0])  # ties
+    logits[1, -1] = logits[2, 0] = 9  # the last expert and the first
+    out, ids, weights = _layer(w).forward(ops.to_device(x), ops.to_device(logits))
+    want, wids, wweights, _ = O.moe_layer(w, x, logits)
+    assert np.array_equal(ids.cpu().numpy().view(np.uint32), wids)
+    assert np.allclose(weights.cpu().numpy(), wweights, rtol=1e-5, atol=0)
+    assert O.rel_l2(out.cpu().numpy(), want) <= REL_L2_F32
+
+
 @pytest.mark.parametrize("inter,pad", [(37, 64), (320, 0), (2880, 0)])
 def test_few_tokens_with_biases_padding_and_absent_slots(inter, pad):
     """MXFP4 with the clamped SwiGLU: odd rows, hidden rows padded with zeros, a slot past the bank giving a NaN row."""
