@@ -104,7 +104,9 @@ struct GmShape {
 // fragments (half of them load addresses worked out in 64 bits, LDS addresses cast through a generic
 // pointer, and M0 saved around every load); loads from a uniform base with 32-bit lane offsets, LDS
 // addresses kept as such and rows that start on 16 bytes (Q4_K) taken as one constant make it about 230
-// and 100. Longer prefetches alone (the rings below, before that) changed nothing. Two 8-wave blocks per
+// and 100 (IQ2_XXS gate/up of 1,500 tokens: 10.4 VALU and 4.0 scalar instructions per MFMA, three pick blocks
+// a stage; 29 % of the waves' time issuing, 36 % on dependencies, 36 % at barriers and for loads, the matrix
+// pipe 21 % busy). Longer prefetches alone (the rings below, before that) changed nothing. Two 8-wave blocks per
 // CU for gate/up instead of one of 16 gave 8 % at 64 tokens. Layers, before and after all of it: 256 IQ2
 // experts, top-8, 2048 x 512, 32 tokens 122 -> 106 us, 64 tokens 157 -> 137, 1,500 tokens 239 -> 230; 128
 // Q4_K experts, 768 x 2048, 256 tokens 155 -> 145; 64 IQ4_XS experts, 16 tokens 121 -> 91; dense Q8_0 4096 x

@@ -86,8 +86,10 @@ struct GateUpShape {
 // of gate and up). Wave 0 routes the token once per block, the token's x stays in registers and the
 // lattice tables in LDS for every item of the block, and an item's weight bytes are requested
 // (unconditionally, from clamped rows and sub-blocks) while the item before it is computed. What
-// bounds it: the dots' VALU work (config 3's shape at 8 tokens: 134M weights of about two
-// instructions each) and the memory round trips of a block's start. With a block per (pick, 8 rows),
+// bounds it: the dots' VALU work and what two waves per SIMD leave uncovered. 256 experts of 2048 x 512, IQ2,
+// top-8, 8 tokens: 134M weights take 8.7M wave instructions on the VALU, four per weight, 14.2 of gate/up's
+// 24.5 us at four cycles each (down 4.3M, 7.0 of 15.2); the waves wait 41% of their time (the block's start,
+// weights), and 64% of the LDS's busy cycles are bank conflicts of the lattice reads, which busy it 25%. With a block per (pick, 8 rows),
 // each wave of it routing the token and reading x for two rows, and down in blocks of 4 rows that
 // each filled the tables, the layer took 77.6 us at 8 tokens and takes 38.8 now; 25.6
 // and 18.9 at 2 tokens; MXFP4 at 2,880 x 2,880, top-4, 8 tokens: 319 and 164 (same output bits but

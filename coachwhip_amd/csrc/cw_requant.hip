@@ -19,7 +19,7 @@
 // the numerator with the exact places where the rounded result steps (Steps); sums that do not
 // change between the fit's rounds are taken once, and the plain shrink has no weights to multiply.
 // VALU-bound: 32 experts of config 5's shape (Q3_K gate and up, Q5_K down, 85 MB in and out) in
-// three launches, 215 -> 109 us (weighted 250 -> 156); about 950 instructions per lane, 2,100 before.
+// three launches, 215 -> 109 us (weighted 250 -> 156); about 960 VALU instructions per lane, 2,100 before.
 #include "cw_common.h"
 #include "cw_requant.h"
 
