@@ -484,7 +484,9 @@ static int grouped_check(int dtype, int64_t n, int64_t k, int64_t n_slots, int64
 // process ends. Every call on a device shares it: the layer's regions are rewritten by each call
 // before they are read, and the sync state is back at zero when each call's kernels end, so a call
 // needs nothing cleared; calls that overlap in time on one device race on it.
-constexpr size_t NOALLOC_SCRATCH_BYTES = CW_MOE_NOALLOC_BYTES;
+// It holds CW_MOE_NOALLOC_BYTES, which the calls are held to with a tile list of piles by slot, and what the
+// tile list of piles by expert may take beyond that (at most 1,024 experts).
+constexpr size_t NOALLOC_SCRATCH_BYTES = CW_MOE_NOALLOC_BYTES + 1024 * sizeof(MfTile);
 static __device__ __align__(256) uint8_t scratch[NOALLOC_SCRATCH_BYTES];
 
 // The device address of this device's copy of `scratch`, looked up once per device (host code
@@ -727,10 +729,15 @@ int cw_moe_layer_noalloc(const cw_moe_desc *desc, const float *x, const float *l
     int rc = check_desc(desc, T);
     if (rc) return rc;
     if (T == 0) return CW_OK;
-    const size_t need = layout(desc, T, false).total;  // (the split GEMMs where their layout fits too)
-    if (need > NOALLOC_SCRATCH_BYTES)
+    const MoeLayout L = layout(desc, T, false);  // (the split GEMMs where their layout fits too)
+    size_t need = L.total;
+    if (L.grouped && piles_by_expert(desc)) {
+        auto list = [&](int piles) { return align256((size_t)max_tiles(T * desc->top_k, piles) * sizeof(MfTile)); };
+        need = need - list(desc->n_experts) + list(desc->n_slots);
+    }
+    if (need > CW_MOE_NOALLOC_BYTES)
         return set_error(CW_EINVAL, "moe noalloc: %d tokens need %zu bytes of scratch, above the %zu the library holds", T, need,
-                         NOALLOC_SCRATCH_BYTES);
+                         CW_MOE_NOALLOC_BYTES);
     void *ws = nullptr;
     if ((rc = noalloc_scratch(&ws))) return rc;
     return moe_layer(desc, x, logits, T, out, ids_out, w_out, missing, ws, NOALLOC_SCRATCH_BYTES, (hipStream_t)stream);

@@ -255,10 +255,12 @@ int cw_moe_layer(const cw_moe_desc *desc, const float *x, const float *logits, i
 /* cw_moe_layer without a workspace, for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid allocation). No counterpart in the
  * reference. Its scratch is one static array per device in the library (CW_MOE_NOALLOC_BYTES,
- * held from the library's load until the process ends); a call whose matvecs' or fp16 GEMMs'
- * workspace is larger is refused with CW_EINVAL (config 3's shape fits about 90 tokens). The call
- * allocates nothing. Every call on a device shares that device's array: calls that overlap in time
- * on one device (on different streams, or from different threads) race and must not be made. Outputs
+ * held from the library's load until the process ends, and 16 KB for the GEMMs' tile lists of
+ * layers with gate or up biases behind a slot table); a call whose matvecs' or fp16 GEMMs'
+ * workspace, with a list as of a layer without those, is larger is refused with CW_EINVAL (config 3's
+ * shape fits about 90 tokens). The call allocates nothing. Every call on a device shares that device's
+ * array: calls that overlap in time on one device (on different streams, or from different threads) race
+ * and must not be made. Outputs
  * equal cw_moe_layer's bit for bit (the same kernels), but for a call that cw_moe_layer runs as GEMMs
  * at f32 accuracy (see there) and whose layout of those does not fit the array: it takes the per-pick
  * matvecs, equal to f32 accuracy. */
